@@ -1476,9 +1476,9 @@ struct hako_gpu_decoder {
 	float *pf_x = nullptr, *pf_xn = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr, *pf_att = nullptr,
 	      *pf_tmp = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_part = nullptr;
 	int8_t *pf_xq = nullptr;                    // q8 rows [chunk][max(d_model, ffn)] and their scales
-	float *pf_xs = nullptr, *pf_esc = nullptr;  // fp16 split of the SwiGLU rows: hi, lo [chunk][ffn], esc[chunk]
-	_Float16 *pf_xh = nullptr, *pf_xl = nullptr;
-	float *pf_sk = nullptr;   // stream-K slots of the down matmul
+	float *pf_xs = nullptr, *pf_esc = nullptr;  // fp16 hi/lo operands of the SwiGLU rows (chunk*ffn*4 bytes), esc[chunk]
+	uint8_t *pf_xh = nullptr;
+	float *pf_sk = nullptr;   // sums of the down matmul's split K
 	size_t pf_sk_floats = 0;
 	int *pf_tok = nullptr, *pf_pos = nullptr;
 	int pf_chunk = 0;   // most tokens per prefill pass
@@ -2048,10 +2048,9 @@ int prefill_alloc(hako_gpu_decoder *d) {
 	HK_ALLOC(d->pf_part, d->pf_part_bytes);
 	HK_ALLOC(d->pf_xq, C * (D > F ? D : F));
 	HK_ALLOC(d->pf_xs, 4 * C * (D > F ? D : F) / 32);
-	HK_ALLOC(d->pf_xh, 2 * C * F);
-	HK_ALLOC(d->pf_xl, 2 * C * F);
+	HK_ALLOC(d->pf_xh, 4 * C * F);
 	HK_ALLOC(d->pf_esc, 4 * C);
-	d->pf_sk_floats = q6k_gemm_sk_floats(q6k_gemm_sk_grid());
+	d->pf_sk_floats = q6k_gemm_sk_max_floats();
 	HK_ALLOC(d->pf_sk, 4 * d->pf_sk_floats);
 	HK_ALLOC(d->pf_tok, 4 * C);
 	HK_ALLOC(d->pf_pos, 4 * C);
@@ -2163,9 +2162,8 @@ int prefill_chunk(hako_gpu_decoder *d, int seq, const int *tokens, int n, int po
 		}
 		// down + residual: h = pf_g
 		if (n > kSkMaxTokens && B.t_down == HAKO_TYPE_Q6_K) {
-			if (int rc = f16_split(d->pf_g, d->pf_xh, d->pf_xl, d->pf_esc, n, F)) return rc;
-			if (int rc = q6k_gemm_split(d->pf_x, B.down, d->pf_xh, d->pf_xl, d->pf_esc, nullptr, n, D, F, true, d->pf_sk,
-			                             d->pf_sk_floats))
+			if (int rc = q6k_gemm_x(d->pf_x, B.down, d->pf_g, d->pf_xh, d->pf_esc, nullptr, n, D, F, true, d->pf_sk,
+			                        d->pf_sk_floats))
 				return rc;
 		} else if (n > kSkMaxTokens && B.t_down == HAKO_TYPE_Q4_K) {
 			if (int rc = hako_gpu_quantize_q8_32(d->pf_g, n, F, d->pf_xq, d->pf_xs)) return rc;

@@ -28,16 +28,17 @@
 // well inside the 1e-5 output tolerance.
 //
 // Tiles: 64 tokens x 64 rows per workgroup of 4 waves (2 x 2, one 32 x 32
-// MFMA tile each); K advances one super-block (Q4_K) or half a super-block
-// (Q6_K) per stage, staged through LDS with the next stage's global loads in
-// flight during the current stage's arithmetic. Workgroup b runs on XCD
-// b % 8, and each XCD is given a contiguous run of tiles in token-tile-major
-// order: the workgroups resident on one XCD share one token tile, whose
-// activations then stay in that XCD's L2.
+// MFMA tile each), K staged through LDS with the next stage's global loads in
+// flight during the current stage's arithmetic; larger tiles where a launch
+// has the work for them (below). Workgroup b runs on XCD b % 8, and each XCD is
+// given a contiguous run of tiles, so that the workgroups resident on one XCD
+// share operands in its L2.
 #include "hako_dev.h"
 #include "hako_rt.h"
 #include "skinny.h"
 #include "q4k_dev.h"
+
+#include <type_traits>
 
 namespace hako {
 namespace {
@@ -560,30 +561,13 @@ __device__ __forceinline__ uint32_t q6_pair(uint32_t v, uint32_t sel) {
 	return __builtin_bit_cast(uint32_t, r);
 }
 
-constexpr int kQ6Stage = 128;        // K per stage: half a super-block
-constexpr int kHPad = kQ6Stage + 8;  // fp16 per staged row (272 B: conflict-free 16-byte reads)
-
-// LDS of one stage buffer of a TN-row tile: activation hi and lo
-// [64][kHPad], q - 32 [TN][kHPad] (fp16), d*sc [8 groups][TN] (fp32).
-__host__ __device__ constexpr size_t q6g_buf_bytes(int tn) {
-	return (size_t)(2 * kTM + tn) * kHPad * 2 + (size_t)8 * tn * 4;
-}
-
-// Tile: 64 tokens x TN rows (64 or 128), one thread per (weight row,
-// quarter of a stage's bytes), waves of one 32 x 32 MFMA tile each (2 token
-// halves x TN/32 row quarters), so every output's arithmetic is the same at
-// both widths. TN = 64: two workgroups per CU, one LDS buffer, two barriers
-// per stage. TN = 128 (DB): one workgroup per CU with the stage buffers
-// double-buffered in LDS, one barrier per stage; a stage's activation then serves twice
-// the rows, so each output needs ~40% fewer staged bytes.
-//
-// Epilogue of a 32 x 32 MFMA tile: lane (li, kh) of wave (wr, wt) holds
-// row n0+32wr+li, tokens m0+32wt+8q4+4kh+r. Every operand load (token
-// scales, bias, the output added to) first, then the stores; lanes past the
-// rows or tokens use an offset past the stream.
-__device__ __forceinline__ void q6g_epilogue(const v16f &acc, int m0, int n0, int wr, int wt, int li, int kh, int M,
-                                             int N, float *y, const float *esc, const float *bias, int add) {
-	const int row = n0 + 32 * wr + li;
+// Epilogue of a 32 x 32 MFMA tile at token m0, row n0: lane (li, kh) holds
+// row n0+li, tokens m0+8q4+4kh+r. Every operand load (token scales, bias, the
+// output added to) first, then the stores; lanes past the rows or tokens use
+// an offset past the stream.
+__device__ __forceinline__ void q6g_epilogue(const v16f &acc, int m0, int n0, int li, int kh, int M, int N, float *y,
+                                             const float *esc, const float *bias, int add) {
+	const int row = n0 + li;
 	const bool rok = row < N;
 	const __amdgpu_buffer_rsrc_t yrs = stream_rsrc(y, (uint32_t)M * (uint32_t)N * 4u);
 	const __amdgpu_buffer_rsrc_t ars = stream_rsrc(y, add ? (uint32_t)M * (uint32_t)N * 4u : 0u);
@@ -594,7 +578,7 @@ __device__ __forceinline__ void q6g_epilogue(const v16f &acc, int m0, int n0, in
 	float ev[16], ov[16];
 #pragma unroll
 	for (int u = 0; u < 16; u++) {
-		const int tok = m0 + 32 * wt + 8 * (u >> 2) + 4 * kh + (u & 3);
+		const int tok = m0 + 8 * (u >> 2) + 4 * kh + (u & 3);
 		const bool ok = rok && tok < M;
 		off[u] = ok ? 4u * ((uint32_t)tok * N + row) : kBufNone;
 		ev[u] = ld_f32(ers, ok ? 4u * tok : kBufNone);
@@ -607,26 +591,36 @@ __device__ __forceinline__ void q6g_epilogue(const v16f &acc, int m0, int n0, in
 	}
 }
 
+constexpr int kQ6Stage = 128;        // K per stage: half a super-block
+constexpr int kHPad = kQ6Stage + 8;  // fp16 per staged row (272 B: conflict-free 16-byte reads)
+
+// ── Q6_K x fp32, 64- and 128-row tiles ──
 //
-// SK (stream-K, with DB): the grid's G workgroups split the launch's
-// tiles x super-blocks evenly, workgroup v (its place in the XCD-contiguous
-// order) taking units [v·U/G, (v+1)·U/G) of the U = tiles·NB in tile order.
-// (Used when tiles < G, so a range is no longer than a tile and meets at
-// most two tiles.) The workgroup leaves
-// each tile's sums, unscaled, in its slot v·2 + (first tile ? 0 : 1) of
-// `skp` (the thread's 16 sums side by side), and q6k_gemm_sk_fixup_kernel
-// adds a tile's slots in workgroup order and applies the epilogue. With 224
-// tiles of 128 rows on 256 CUs (7B down over 512 tokens) every CU works
-// instead of 7 in 8.
-template <int TN, bool DB, bool SK = false>
+// For short K (q6k_gemm_plan): their start-up is the shortest (10 against 14
+// us at 512 x 64 x 256 with the split of the activations, 25 against 34 at
+// 512 x 4096 x 1024), their cost per super-block the highest (273 against 192 us
+// at 512 x 3584 x 18944).
+//
+// LDS of one stage buffer of a TN-row tile: activation hi and lo
+// [64][kHPad], q - 32 [TN][kHPad] (fp16), d*sc [8 groups][TN] (fp32).
+__host__ __device__ constexpr size_t q6g_buf_bytes(int tn) {
+	return (size_t)(2 * kTM + tn) * kHPad * 2 + (size_t)8 * tn * 4;
+}
+
+// Tile: 64 tokens x TN rows (64 or 128), one thread per (weight row,
+// quarter of a stage's bytes), waves of one 32 x 32 MFMA tile each (2 token
+// halves x TN/32 row quarters). TN = 64: two workgroups per CU, one LDS
+// buffer, two barriers per stage. TN = 128 (DB): one workgroup per CU with
+// the stage buffers double-buffered in LDS, one barrier per stage; a stage's
+// activation then serves twice the rows.
+template <int TN, bool DB>
 __global__ __launch_bounds__(4 * TN, DB ? 1 : 2) void q6k_gemm_kernel(const uint8_t *__restrict__ w,
                                                                      const _Float16 *__restrict__ xh,
                                                                      const _Float16 *__restrict__ xl,
                                                                      const float *__restrict__ esc,
                                                                      const float *__restrict__ bias,
                                                                      float *__restrict__ y, int M, int N, int K,
-                                                                     int add, int gm, float *__restrict__ skp) {
-	static_assert(!SK || DB, "stream-K runs the double-buffered tiles");
+                                                                     int add, int gm) {
 	constexpr int T = 4 * TN;           // threads
 	constexpr int PA = kTM * 16 / T;    // activation pieces (16 B) per thread, hi and lo each
 	constexpr int RQ = TN / 32;         // row quarters (waves per token half)
@@ -647,23 +641,11 @@ __global__ __launch_bounds__(4 * TN, DB ? 1 : 2) void q6k_gemm_kernel(const uint
 
 	const int mtiles = (M + kTM - 1) / kTM, ntiles = (N + TN - 1) / TN;
 	const int NB = K >> 8;
-	// SK: this workgroup's units (super-blocks of tiles in tile order)
-	int64_t u_beg = 0, u_end = 0;
-	int tile, vpos = 0;
-	if constexpr (SK) {
-		vpos = xcd_tile(blockIdx.x, gridDim.x);
-		const int64_t U = (int64_t)mtiles * ntiles * NB;
-		u_beg = (int64_t)vpos * U / gridDim.x;
-		u_end = (int64_t)(vpos + 1) * U / gridDim.x;
-		if (u_end <= u_beg) return;
-		tile = (int)(u_beg / NB);
-	} else {
-		tile = xcd_tile(blockIdx.x, mtiles * ntiles);
-		if (tile >= mtiles * ntiles) return;
-	}
+	const int tile = xcd_tile(blockIdx.x, mtiles * ntiles);
+	if (tile >= mtiles * ntiles) return;
 	int mt, nt;
 	tile_mn(tile, ntiles, gm, mt, nt);
-	int m0 = mt * kTM, n0 = nt * TN;
+	const int m0 = mt * kTM, n0 = nt * TN;
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int wr = wave % RQ, wt = wave / RQ, li = lane & 31, kh = lane >> 5;
 	const uint32_t rb = (uint32_t)NB * kQ6Bytes;
@@ -688,14 +670,13 @@ __global__ __launch_bounds__(4 * TN, DB ? 1 : 2) void q6k_gemm_kernel(const uint
 		uint32_t sc, d;
 	};
 	const int NSt = NB * 2;
-	int s_end = NSt;   // stages past it load nothing
 	// unconditional: a stage past the last loads nothing (out-of-range offsets)
 	auto load_acts = [&](Acts &r, int st) {
 		const uint32_t k0 = (uint32_t)kQ6Stage * st;
 #pragma unroll
 		for (int u = 0; u < PA; u++) {
 			const int c = tid + T * u, tok = c >> 4, piece = c & 15;
-			const bool on = st < s_end && m0 + tok < M;
+			const bool on = st < NSt && m0 + tok < M;
 			const uint32_t off = on ? 2u * ((uint32_t)(m0 + tok) * K + k0 + 8u * piece) : kBufNone;
 			r.h[u] = ld_b128(hrs, off);
 			r.l[u] = ld_b128(lrs, off);
@@ -703,7 +684,7 @@ __global__ __launch_bounds__(4 * TN, DB ? 1 : 2) void q6k_gemm_kernel(const uint
 	};
 	auto load_wts = [&](Wts &r, int st) {
 		const int kb = st >> 1, n = st & 1;
-		const bool on = st < s_end && n0 + wrow < N;
+		const bool on = st < NSt && n0 + wrow < N;
 		const uint32_t blk = on ? (uint32_t)(n0 + wrow) * rb + (uint32_t)kb * kQ6Bytes : kBufNone;
 		const uint32_t oql = 64u * n + 16u * part, oqh = 128u + 32u * n + 16u * (part & 1);
 		r.ql[0] = ld_b64(wrs, blk + oql);
@@ -801,91 +782,396 @@ __global__ __launch_bounds__(4 * TN, DB ? 1 : 2) void q6k_gemm_kernel(const uint
 		const View v1 = view(1);
 		Acts aa, ab;
 		Wts wts;
-		// stages [sa, sb) of the current tile
-		auto pipeline = [&](int sa, int sb) {
-			s_end = sb;
-			load_acts(aa, sa);
-			load_wts(wts, sa);
-			load_acts(ab, sa + 1);
-			for (int st = sa; st < sb; st += 2) {
-				store_acts(aa, v0);
-				store_wts(wts, v0);
-				__syncthreads();
-				load_wts(wts, st + 1);
-				load_acts(aa, st + 2);
-				compute(v0);
-				store_acts(ab, v1);
-				store_wts(wts, v1);
-				__syncthreads();
-				load_wts(wts, st + 2);
-				load_acts(ab, st + 3);
-				compute(v1);
-			}
-		};
-		if constexpr (SK) {
-			// one or two tiles: each piece's sums to its slot, then the next
-			// tile (the buffers' last readers passed a barrier since: v0 was
-			// read before the barrier that followed the stores of v1, and v1
-			// is next written after the barrier that follows those of v0)
-			const int first = tile;
-			for (;;) {
-				const int64_t t0u = (int64_t)tile * NB;
-				const int ka = (int)(u_beg > t0u ? u_beg - t0u : 0);
-				const int kb = (int)(u_end < t0u + NB ? u_end - t0u : NB);
-				pipeline(2 * ka, 2 * kb);
-				float4 *dst = (float4 *)(skp + ((size_t)(2 * vpos + (tile == first ? 0 : 1)) * T + tid) * 16);
-#pragma unroll
-				for (int q = 0; q < 4; q++) dst[q] = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-				if (t0u + NB >= u_end) return;
-				acc = zero;
-				tile++;
-				tile_mn(tile, ntiles, gm, mt, nt);
-				m0 = mt * kTM;
-				n0 = nt * TN;
-			}
-		} else {
-			pipeline(0, NSt);
+		load_acts(aa, 0);
+		load_wts(wts, 0);
+		load_acts(ab, 1);
+		for (int st = 0; st < NSt; st += 2) {
+			store_acts(aa, v0);
+			store_wts(wts, v0);
+			__syncthreads();
+			load_wts(wts, st + 1);
+			load_acts(aa, st + 2);
+			compute(v0);
+			store_acts(ab, v1);
+			store_wts(wts, v1);
+			__syncthreads();
+			load_wts(wts, st + 2);
+			load_acts(ab, st + 3);
+			compute(v1);
 		}
 	}
-	q6g_epilogue(acc, m0, n0, wr, wt, li, kh, M, N, y, esc, bias, add);
+	q6g_epilogue(acc, m0 + 32 * wt, n0 + 32 * wr, li, kh, M, N, y, esc, bias, add);
 }
 
-// Sums of the stream-K pieces of tile blockIdx.x (q6k_gemm_kernel<128, true,
-// true>: same threads, same slots), added in workgroup order, that is in
-// order of K, and the GEMM's epilogue.
-__global__ __launch_bounds__(512) void q6k_gemm_sk_fixup_kernel(const float *__restrict__ skp,
-                                                                const float *__restrict__ esc,
-                                                                const float *__restrict__ bias, float *__restrict__ y,
-                                                                int M, int N, int NB, int G, int gm, int add) {
-	constexpr int TN = 128, T = 4 * TN, RQ = TN / 32;
-	const int mtiles = (M + kTM - 1) / kTM, ntiles = (N + TN - 1) / TN;
-	const int tile = blockIdx.x;
-	const int64_t U = (int64_t)mtiles * ntiles * NB;
-	auto start = [&](int v) -> int64_t { return (int64_t)v * U / G; };
-	const int64_t a = (int64_t)tile * NB, b = a + NB;
-	int v = (int)(a * G / U);   // the workgroup holding unit a
-	while (start(v + 1) <= a) v++;
-	while (v > 0 && start(v) > a) v--;
-	const int tid = threadIdx.x;
-	v16f acc = {};
-	for (; v < G && start(v) < b; v++) {
-		const int64_t s0 = start(v), s1 = start(v + 1);
-		if (s1 <= s0 || s1 <= a) continue;
-		const int which = s0 / NB == tile ? 0 : 1;   // the tile is the workgroup's first or second
-		const float4 *src = (const float4 *)(skp + ((size_t)(2 * v + which) * T + tid) * 16);
+// ── Q6_K x fp32, 256-row tiles ──
+//
+// What bounds it: per 32 x 32 x 16 product pair (hi, lo) 64 cycles of matrix
+// core stand against 64 of the fold's FMAs and ~20 of the weights' unpacking
+// on the vector ALUs, and the operands have to reach four SIMDs through an
+// LDS and an L1 that give 64 bytes a cycle each (measured, 16-byte accesses).
+// With both operands in LDS and one 32 x 32 tile per wave (the 64 x 64 tiles
+// above) a pair takes 3 KB of LDS: 192 cycles of its CU for four pairs' 64.
+// So a wave takes 32 tokens x 32 RT rows; the weights, unpacked once for the
+// workgroup, come from LDS (1 KB per pair, and the stores), and the
+// activations, laid out by f16_pack_kernel so that an operand is one contiguous
+// KB, straight from memory: the workgroup's waves read the same ones at
+// about the same time, from the CU's L1 (2 / RT KB per pair). 64 x 64 per
+// wave, with twice the L1 and half the LDS bytes, measured 209 us at
+// 512 x 3584 x 18944 where this split takes 195, and activations through LDS
+// as well 206.
+// Workgroup: TM / 32 token tiles x 8 / RT groups of 32 RT rows, 256 rows in all.
+// K advances 64 wide per stage (the low, then the high nibbles of a half
+// super-block), the weights double-buffered in LDS with one barrier per stage.
+//
+// Few tiles leave CUs idle, so K is split over `ks` workgroups per tile. They
+// run split by split: the workgroups of an XCD take the same range of K at the
+// same time, and share its weights and activations in that XCD's L2. (Even
+// shares of the tiles' super-blocks, stream-K, keep 256 instead of 224 CUs
+// busy at 512 x 3584 x 18944, but every workgroup then stands at a K of its
+// own and reads from beyond L2: 11.6 against 9.8 us per super-block.) With ks > 1 a workgroup
+// leaves its sums, unscaled, in slot `v` of `skp`, and q6k_gemm_fix_kernel
+// adds a tile's in order of K.
+constexpr int kQ6TN = 256;                // weight rows per tile
+constexpr int kQ6T = 512;                 // threads
+constexpr int kQ6SK = 64;                 // K per stage
+constexpr int kQ6RowB = 2 * kQ6SK + 16;   // bytes per staged row (conflict-free 16-byte accesses)
+constexpr int kQ6BufB = kQ6TN * kQ6RowB + 4 * kQ6TN * 4;   // a stage buffer: rows, d*sc [4 groups][256]
+
+__host__ __device__ constexpr size_t q6w_slot(int tm) { return (size_t)tm * kQ6TN; }   // floats per slot
+
+template <int TM>
+__global__ __launch_bounds__(kQ6T, 2) void q6k_gemm_wide_kernel(const uint8_t *__restrict__ w,
+                                                             const uint8_t *__restrict__ xp,
+                                                             const float *__restrict__ esc,
+                                                             const float *__restrict__ bias, float *__restrict__ y,
+                                                             int M, int N, int K, int add, int gm, int ks,
+                                                             float *__restrict__ skp) {
+	constexpr int RT = TM / 32;            // 32-row tiles per wave; TM / 32 token tiles x 8 / RT row groups of waves
+	__shared__ __align__(16) uint8_t lds[2 * kQ6BufB];
+	const int mtiles = (M + TM - 1) / TM, ntiles = (N + kQ6TN - 1) / kQ6TN;
+	const int NB = K >> 8;
+	const int tiles = mtiles * ntiles, vpos = xcd_tile(blockIdx.x, tiles * ks);
+	if (vpos >= tiles * ks) return;
+	const int split = vpos / tiles;
+	int mt, nt;
+	tile_mn(vpos - split * tiles, ntiles, gm, mt, nt);
+	const int m0 = mt * TM, n0 = nt * kQ6TN;
+	const int ka = (int)((int64_t)split * NB / ks), kb = (int)((int64_t)(split + 1) * NB / ks);   // super-blocks
+	const int s_end = 4 * kb, g_end = 16 * kb;   // stages past s_end load nothing, groups past g_end repeat the last
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int wr = wave % (8 / RT), wt = wave / (8 / RT), li = lane & 31, kh = lane >> 5;
+	const uint32_t rb = (uint32_t)NB * kQ6Bytes;
+	const __amdgpu_buffer_rsrc_t wrs = stream_rsrc(w, rb * (uint32_t)N);
+
+	// Weights: thread (row tid/2, h = tid%2) takes ql bytes [64n + 32h, +32) and
+	// qh bytes [128 + 32n, +32) of half n, i.e. K 32h.. (low nibbles, qh bits
+	// 2h) and 64 + 32h.. (high nibbles, qh bits 4 + 2h) of the half: 32
+	// weights, two scale groups, of each of its two stages.
+	const int wrow = tid >> 1, h = tid & 1;
+	struct Wts {
+		uint4 ql[2], qh[2], sc;   // sc: the block's 16 scales
+		uint32_t d;
+	};
+	Wts wa;
+	auto wts_block = [&](int st) {   // the thread's block of stage st (even)
+		return ((uint32_t)(n0 + wrow) * rb + (uint32_t)(st >> 2) * kQ6Bytes) | (n0 + wrow < N ? 0u : kBufNone) |
+		       ((uint32_t)((s_end - 1 - st) >> 31) & kBufNone);
+	};
+	auto load_piece = [&](uint32_t blk, int n, int j) {   // 16 of its bytes of ql and qh of half n
+		wa.ql[j] = ld_b128(wrs, blk + 64u * n + 32u * h + 16u * j);
+		wa.qh[j] = ld_b128(wrs, blk + 128u + 32u * n + 16u * j);
+	};
+	auto load_scales = [&](uint32_t blk) {
+		wa.sc = ld_b128(wrs, blk + 192u);
+		wa.d = ld_b16(wrs, blk + 208u);
+	};
+	// dword i (of 8) of the thread's stage: four weights of stage s (0 low
+	// nibbles, 1 high) as two fp16 pairs; every second one completes 16 bytes
+	uint32_t o[4];
+	auto conv_wts = [&](uint8_t *buf, int s, int i) {
+		const uint4 q4 = wa.ql[i >> 2], h4 = wa.qh[i >> 2];
+		const uint32_t ql = (i & 3) == 0 ? q4.x : (i & 3) == 1 ? q4.y : (i & 3) == 2 ? q4.z : q4.w;
+		const uint32_t qh = (i & 3) == 0 ? h4.x : (i & 3) == 1 ? h4.y : (i & 3) == 2 ? h4.z : h4.w;
+		const uint32_t v = s == 0 ? (((qh << (4 - 2 * h)) & 0x30303030u) | (ql & 0x0F0F0F0Fu))
+		                          : (((qh >> (2 * h)) & 0x30303030u) | ((ql >> 4) & 0x0F0F0F0Fu));
+		o[2 * (i & 1)] = q6_pair(v, 0x04010400u);
+		o[2 * (i & 1) + 1] = q6_pair(v, 0x04030402u);
+		if (i & 1) *(uint4 *)(buf + wrow * kQ6RowB + 64 * h + 16 * (i >> 1)) = make_uint4(o[0], o[1], o[2], o[3]);
+	};
+	// the thread's scales 8n + 4s + 2h, +1 of stage s of half n
+	auto conv_scales = [&](uint8_t *buf, int n, int s) {
+		float *dsc = (float *)(buf + kQ6TN * kQ6RowB);
+		const float d = f16_to_f32(wa.d);
+		const uint32_t sc = (n == 0 ? (s == 0 ? wa.sc.x : wa.sc.y) : (s == 0 ? wa.sc.z : wa.sc.w)) >> (16 * h);
+		dsc[(2 * h) * kQ6TN + wrow] = d * (float)(int8_t)(sc & 0xFFu);
+		dsc[(2 * h + 1) * kQ6TN + wrow] = d * (float)(int8_t)((sc >> 8) & 0xFFu);
+	};
+
+	// Activations: this wave's token tile in xp (the last tile of the launch
+	// holds th < 32 tokens; lanes past them repeat its last one, and a wave
+	// past the tokens the last tile: computed and not stored).
+	const int tt = min(m0 / 32 + wt, (M - 1) / 32);
+	const uint32_t th = (uint32_t)min(32, M - 32 * tt);
+	const uint32_t av = 16u * ((uint32_t)kh * th + min((uint32_t)li, th - 1));   // the lane's 16 bytes of a group
+	const __amdgpu_buffer_rsrc_t ars = stream_rsrc(uniform_ptr(xp + (size_t)tt * 128 * K), th * (uint32_t)K * 4u);
+	v8h ah[2], al[2];   // two groups in flight
+	auto load_acts = [&](int g) {
+		const int go = (int)(th * 64u) * min(g, g_end - 1);
+		ah[g & 1] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(ars, (int)av, go, 0));
+		al[g & 1] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(ars, (int)av, go + (int)th * 32, 0));
+	};
+
+	v16f acc[RT] = {};
+	const v16f zero = {};
+	// One stage (half n; S = 0 from the low nibbles in buf, 1 from the high
+	// ones) as NS steps (scale group g, row tile r). Step k's two products run on
+	// the matrix cores while the vector ALUs fold step k - 1's and unpack a
+	// slice of the next stage's weights into `obuf`. Everything is spread over
+	// the steps: a wave issues in order, so products in a row hold its folds
+	// back, and loads in a row wait for the memory pipes. The activations are
+	// reloaded (two groups ahead) once their products are issued, and a piece of
+	// the weights (S = 0: from half st + 2) once both its nibbles are unpacked.
+	auto compute = [&](const uint8_t *buf, uint8_t *obuf, auto nc, auto sc, int st) {
+		constexpr int n = decltype(nc)::value, S = decltype(sc)::value, NS = 4 * RT, CS = NS / 8;
+		const uint8_t *wp = buf + (32 * RT * wr + li) * kQ6RowB + 16 * kh;
+		const float *dsc = (const float *)(buf + kQ6TN * kQ6RowB) + 32 * RT * wr + li;
+		const uint32_t nblk = S == 0 ? wts_block(st + 2) : 0u;
+		v8h b[2][RT];
+		float s[2][RT];
+		v16f p[2];
+		float ps[2];   // the scale of the products in p
+		auto read = [&](int g, int r) {
+			b[g & 1][r] = *(const v8h *)(wp + r * 32 * kQ6RowB + 32 * g);
+			s[g & 1][r] = dsc[g * kQ6TN + 32 * r];
+		};
 #pragma unroll
-		for (int q = 0; q < 4; q++) {
-			const float4 t = src[q];
-			acc[4 * q] += t.x;
-			acc[4 * q + 1] += t.y;
-			acc[4 * q + 2] += t.z;
-			acc[4 * q + 3] += t.w;
+		for (int r = 0; r < RT; r++) read(0, r);
+#pragma unroll
+		for (int k = 0; k <= NS; k++) {
+			const int g = k / RT, r = k % RT;
+			if (g + 1 < 4) read(g + 1, r);
+			if (k < NS) {
+				ps[k & 1] = s[g & 1][r];
+				p[k & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[g & 1], b[g & 1][r], zero, 0, 0, 0);
+				p[k & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[g & 1], b[g & 1][r], p[k & 1], 0, 0, 0);
+				if (r == RT - 1) load_acts(4 * st + g + 2);
+				if (k % CS == 0) conv_wts(obuf, 1 - S, k / CS);
+				if (k == NS - 2) conv_scales(obuf, S == 0 ? n : 1 - n, 1 - S);
+				if (S == 0 && k == 4 * CS) load_piece(nblk, 1 - n, 0);
+				if (S == 0 && k == NS - 1) {
+					load_piece(nblk, 1 - n, 1);
+					if (n == 1) load_scales(nblk);
+				}
+			}
+			if (k > 0) {
+				const int f = k - 1;
+#pragma unroll
+				for (int v = 0; v < 16; v++) acc[f % RT][v] = __builtin_fmaf(p[f & 1][v], ps[f & 1], acc[f % RT][v]);
+			}
+			if (k < NS) {
+#pragma unroll
+				for (int i = 0; i < 2; i++) {
+					__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+					__builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+					__builtin_amdgcn_sched_group_barrier(0x080, 1, 0);
+					__builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+					__builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+				}
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	};
+
+	uint8_t *const b0 = lds, *const b1 = lds + kQ6BufB;
+	{
+		const uint32_t blk = wts_block(4 * ka);
+		load_piece(blk, 0, 0);
+		load_piece(blk, 0, 1);
+		load_scales(blk);
+	}
+	load_acts(16 * ka);
+	load_acts(16 * ka + 1);
+	// Stage st is in buffer st % 2, stored before the barrier that ends
+	// stage st - 1, after the barrier that ended the buffer's last reader.
+	// #pragma unroll
+	for (int i = 0; i < 8; i++) conv_wts(b0, 0, i);
+	conv_scales(b0, 0, 0);
+	__syncthreads();
+	constexpr std::integral_constant<int, 0> c0{};
+	constexpr std::integral_constant<int, 1> c1{};
+	for (int st = 4 * ka; st < s_end; st += 4) {
+		compute(b0, b1, c0, c0, st);
+		__syncthreads();
+		compute(b1, b0, c0, c1, st + 1);
+		__syncthreads();
+		compute(b0, b1, c1, c0, st + 2);
+		__syncthreads();
+		compute(b1, b0, c1, c1, st + 3);
+		__syncthreads();
+	}
+	if (ks == 1) {
+#pragma unroll
+		for (int r = 0; r < RT; r++)
+			q6g_epilogue(acc[r], m0 + 32 * wt, n0 + 32 * (RT * wr + r), li, kh, M, N, y, esc, bias, add);
+	} else {
+		float4 *dst = (float4 *)(skp + (size_t)vpos * q6w_slot(TM)) + tid;
+#pragma unroll
+		for (int r = 0; r < RT; r++)
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+				dst[(size_t)(r * 4 + q) * kQ6T] =
+				    make_float4(acc[r][4 * q], acc[r][4 * q + 1], acc[r][4 * q + 2], acc[r][4 * q + 3]);
+	}
+}
+
+// The sums of a tile's ks workgroups of q6k_gemm_wide_kernel, added in order
+// of K, and the epilogue: workgroup (tile, one of its 4 RT float4 of every
+// thread); a thread's four sums are tokens 8q + 4kh .. +4 of one row. Eight
+// loads are in flight at a time.
+template <int TM>
+__global__ __launch_bounds__(kQ6T) void q6k_gemm_fix_kernel(const float *__restrict__ skp,
+                                                            const float *__restrict__ esc,
+                                                            const float *__restrict__ bias, float *__restrict__ y,
+                                                            int M, int N, int tiles, int ks, int gm, int add) {
+	constexpr int RT = TM / 32;
+	const int ntiles = (N + kQ6TN - 1) / kQ6TN;
+	const int tile = blockIdx.x / (4 * RT), part = blockIdx.x % (4 * RT);
+	const int tid = threadIdx.x;
+	const float4 *src = (const float4 *)(skp + (size_t)tile * q6w_slot(TM)) + (size_t)part * kQ6T + tid;
+	const size_t step = (size_t)tiles * q6w_slot(TM) / 4;
+	float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	for (int v = 0; v < ks; v += 8) {
+		float4 t[8];
+#pragma unroll
+		for (int i = 0; i < 8; i++) t[i] = src[step * min(v + i, ks - 1)];
+#pragma unroll
+		for (int i = 0; i < 8; i++) {
+			const bool on = v + i < ks;
+			acc.x += on ? t[i].x : 0.0f;
+			acc.y += on ? t[i].y : 0.0f;
+			acc.z += on ? t[i].z : 0.0f;
+			acc.w += on ? t[i].w : 0.0f;
 		}
 	}
 	int mt, nt;
 	tile_mn(tile, ntiles, gm, mt, nt);
-	const int lane = tid & 63, wave = tid >> 6;
-	q6g_epilogue(acc, mt * kTM, nt * TN, wave % RQ, wave / RQ, lane & 31, lane >> 5, M, N, y, esc, bias, add);
+	const int lane = tid & 63, wave = tid >> 6, wr = wave % (8 / RT), wt = wave / (8 / RT);
+	const int q = part & 3, r = part >> 2;
+	const int row = nt * kQ6TN + 32 * (RT * wr + r) + (lane & 31);
+	const int tok0 = mt * TM + 32 * wt + 8 * q + 4 * (lane >> 5);
+	if (row >= N) return;
+	const float bv = bias ? bias[row] : 0.0f;
+	const float f[4] = {acc.x, acc.y, acc.z, acc.w};
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		if (tok0 + i >= M) break;
+		float *o = y + (size_t)(tok0 + i) * N + row;
+		const float u = f[i] * esc[tok0 + i] + bv;
+		*o = add ? *o + u : u;
+	}
+}
+
+// The fp16 hi/lo split of f16_split_kernel, laid out as q6k_gemm_wide_kernel's
+// operands: xp holds the 32-token tiles one after another, each as K/16
+// groups of [hi: 2 k halves][lo: 2 k halves] x th tokens x 8 values, th = 32
+// but for the last tile (M K 4 bytes in all).
+__device__ __forceinline__ void f16_put(uint8_t *xp, int tok, int k8, int M, int K, const float4 &v0, const float4 &v1,
+                                        float sc) {
+	const int tt = tok >> 5, th = min(32, M - 32 * tt);
+	const float f[8] = {v0.x * sc, v0.y * sc, v0.z * sc, v0.w * sc, v1.x * sc, v1.y * sc, v1.z * sc, v1.w * sc};
+	v8h hi, lo;
+#pragma unroll
+	for (int i = 0; i < 8; i++) {
+		hi[i] = (_Float16)f[i];
+		lo[i] = (_Float16)(f[i] - (float)hi[i]);
+	}
+	uint8_t *o = xp + (size_t)tt * 128 * K + (size_t)(k8 >> 1) * th * 64 + 16 * ((k8 & 1) * th + (tok & 31));
+	*(v8h *)o = hi;
+	*(v8h *)(o + 32 * th) = lo;
+}
+
+__device__ __forceinline__ float amax4(const float4 &q) {
+	return __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(q.x), __builtin_fabsf(q.y)),
+	                       __builtin_fmaxf(__builtin_fabsf(q.z), __builtin_fabsf(q.w)));
+}
+
+// Rows of up to kPackK values in one launch: a workgroup holds 8 tokens (a
+// thread 8 values of one, 8 neighbouring lanes the 8 tokens, so that an operand's
+// pieces are written 128 bytes at a time). Wider rows would leave most CUs idle
+// (18944 values, 512 tokens: 64 workgroups of 600 KB) and take two launches:
+// f16_esc_kernel a row's power of two, f16_pack_kernel the operands.
+constexpr int kEscT = 1024, kPackK = 4096;
+template <int T, int PP>   // PP pieces of 8 values per thread: rows of up to T PP values
+__global__ __launch_bounds__(T) void f16_pack8_kernel(const float *__restrict__ x, float *__restrict__ esc,
+                                                          uint8_t *__restrict__ xp, int M, int K) {
+	__shared__ float red[T / kWave][8];
+	const int tok = blockIdx.x * 8 + (threadIdx.x & 7), k0 = threadIdx.x >> 3;
+	const float *xr = x + (size_t)min(tok, M - 1) * K;
+	float4 v[PP][2];
+	float a = 0.0f;
+#pragma unroll
+	for (int u = 0; u < PP; u++) {   // pieces past the row repeat its last
+		const int k8 = min(k0 + T / 8 * u, K / 8 - 1);
+		v[u][0] = *(const float4 *)(xr + 8 * k8);
+		v[u][1] = *(const float4 *)(xr + 8 * k8 + 4);
+	}
+#pragma unroll
+	for (int u = 0; u < PP; u++) a = __builtin_fmaxf(a, __builtin_fmaxf(amax4(v[u][0]), amax4(v[u][1])));
+	a = __builtin_fmaxf(a, __shfl_xor(a, 8));
+	a = __builtin_fmaxf(a, __shfl_xor(a, 16));
+	a = __builtin_fmaxf(a, __shfl_xor(a, 32));
+	if ((threadIdx.x & 63) < 8) red[threadIdx.x >> 6][threadIdx.x & 7] = a;
+	__syncthreads();
+	a = 0.0f;
+#pragma unroll
+	for (int w = 0; w < T / kWave; w++) a = __builtin_fmaxf(a, red[w][threadIdx.x & 7]);
+	if (tok >= M) return;
+	const int e = f16_split_exp(a);
+	if (threadIdx.x < 8) esc[tok] = __builtin_ldexpf(1.0f, e);
+	const float sc = __builtin_ldexpf(1.0f, -e);
+#pragma unroll
+	for (int u = 0; u < PP; u++) {
+		const int k8 = k0 + T / 8 * u;
+		if (k8 < K / 8) f16_put(xp, tok, k8, M, K, v[u][0], v[u][1], sc);
+	}
+}
+
+__global__ __launch_bounds__(kEscT) void f16_esc_kernel(const float *__restrict__ x, float *__restrict__ esc, int K) {
+	__shared__ float red[kEscT / kWave];
+	const float *xr = x + (size_t)blockIdx.x * K;
+	float a = 0.0f;
+	for (int i0 = threadIdx.x * 4; i0 < K; i0 += kEscT * 4 * 4) {
+		float4 v[4];
+#pragma unroll
+		for (int u = 0; u < 4; u++) v[u] = *(const float4 *)(xr + min(i0 + kEscT * 4 * u, K - 4));   // repeats are harmless
+#pragma unroll
+		for (int u = 0; u < 4; u++) a = __builtin_fmaxf(a, amax4(v[u]));
+	}
+	a = wave_max(a);
+	if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		for (int i = 1; i < kEscT / kWave; i++) a = __builtin_fmaxf(a, red[i]);
+		esc[blockIdx.x] = __builtin_ldexpf(1.0f, f16_split_exp(a));
+	}
+}
+
+// Workgroup (32-token tile, 256-value block).
+__global__ __launch_bounds__(256) void f16_pack_kernel(const float *__restrict__ x, const float *__restrict__ esc,
+                                                       uint8_t *__restrict__ xp, int M, int K) {
+#pragma unroll
+	for (int u = 0; u < 4; u++) {
+		// token c % 8 + 8 (c / 256) of the tile, values 8 (c/8 % 32).. of the block
+		const int c = threadIdx.x + 256 * u, tok = 32 * blockIdx.x + (c & 7) + 8 * (c >> 8);
+		const int k8 = 32 * blockIdx.y + ((c >> 3) & 31);
+		if (tok >= M) continue;
+		const float *xr = x + (size_t)tok * K + 8 * k8;
+		const float4 v0 = *(const float4 *)xr, v1 = *(const float4 *)(xr + 4);
+		// 2^-e of esc = 2^e (e in -126..127)
+		const int e = (int)((__builtin_bit_cast(uint32_t, esc[tok]) >> 23) & 0xFFu) - 127;
+		f16_put(xp, tok, k8, M, K, v0, v1, __builtin_ldexpf(1.0f, -e));
+	}
 }
 
 // Split-K partials of the skinny matmuls (workspace slot 5).
@@ -901,8 +1187,8 @@ int skinny_split_workspace(size_t floats, float **part) {
 // Token tiles per XCD group (tile_mn): the divisor of the token tiles that
 // minimizes what one XCD reads, gm token tiles of act_tile bytes each plus
 // its share of the row tiles of w_tile bytes each.
-int gemm_gm(int M, int N, double act_tile, double w_tile, int tn = kTN) {
-	const int mtiles = (M + kTM - 1) / kTM, ntiles = (N + tn - 1) / tn;
+int gemm_gm(int M, int N, double act_tile, double w_tile, int tn = kTN, int tm = kTM) {
+	const int mtiles = (M + tm - 1) / tm, ntiles = (N + tn - 1) / tn;
 	const double per = (double)mtiles * ntiles / kXcds;
 	int best = 1;
 	double best_bytes = 1e300;
@@ -926,16 +1212,10 @@ int gemm_grid(int M, int N, int tn = kTN) {
 // Q4_K GEMM with K <= 3840: the resident-token-tile kernel (1) or the tiled
 // one (0); a launch-shape knob
 int g_q4_gemm_res = 1;
-// Q6_K GEMM tile width: -1 by shape, else 64 or 128 rows (a launch-shape knob;
-// the outputs do not depend on it)
-int g_q6_gemm_tn = -1;
-// Stream-K for 128-row tile counts below the workgroups of one round: in the
-// decoder's prompt pass (1), there and in the standalone matmul entry points
-// (2), or never (0). Measured on 512x3584x18944: inside the 7B prompt pass
-// the stream-K kernel and its fixup took 243.8 + 7.0 us against 263.7 us for
-// whole tiles (the pass 18.45 -> 18.12 ms); the same launch repeated back to
-// back, the chip's power limit holding its clocks, 270 against 258 us (with
-// a 3 ms pause before each launch 288 against 300 us).
+// Q6_K GEMM in 256-row tiles of 64 or 128 tokens, or -1: by shape (a
+// launch-shape knob; the outputs of an unsplit K do not depend on it)
+int g_q6_gemm_tm = -1;
+// Split K in the Q6_K GEMM (0: one workgroup per tile)
 int g_q6_gemm_sk = 1;
 
 int check_gemm(const char *what, int m, int n_out, int n_in, size_t row_bytes, const void *w) {
@@ -952,8 +1232,8 @@ int check_gemm(const char *what, int m, int n_out, int n_in, size_t row_bytes, c
 }  // namespace
 
 void q4k_gemm_set_res(int v) { g_q4_gemm_res = v ? 1 : 0; }
-void q6k_gemm_set_tn(int v) { g_q6_gemm_tn = (v == 64 || v == 128) ? v : -1; }
-void q6k_gemm_set_sk(int v) { g_q6_gemm_sk = v < 0 ? 0 : (v > 2 ? 2 : v); }
+void q6k_gemm_set_tn(int v) { g_q6_gemm_tm = (v == 64 || v == 128) ? v : -1; }
+void q6k_gemm_set_sk(int v) { g_q6_gemm_sk = v > 0; }
 
 int q4k_gemm(float *y, const void *w, const int8_t *xq, const float *xs, const float *bias, int m, int n_out,
              int n_in) {
@@ -1028,11 +1308,11 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 	const size_t half_bytes = (size_t)m * n_in * 2, esc_off = 2 * ((half_bytes + 255) & ~(size_t)255);
 	void *ws = nullptr;
 	if (int rc = workspace(3, esc_off + (size_t)m * 4, &ws)) return rc;
-	_Float16 *xh = (_Float16 *)ws;
-	_Float16 *xl = (_Float16 *)((uint8_t *)ws + esc_off / 2);
 	float *esc = (float *)((uint8_t *)ws + esc_off);
-	if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 	if (m <= kSkMaxTokens) {   // a few tokens: the skinny kernel
+		_Float16 *xh = (_Float16 *)ws;
+		_Float16 *xl = (_Float16 *)((uint8_t *)ws + esc_off / 2);
+		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 		SkSegs segs{};
 		segs.n = 1;
 		segs.s[0] = {(const uint8_t *)w, bias, y, 0, n_out, n_out};
@@ -1043,51 +1323,116 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 		return ok();
 	}
 	float *skp = nullptr;
-	size_t skf = 0;
-	if (g_q6_gemm_sk == 2) {   // stream-K slots (workspace slot 6)
-		skf = q6k_gemm_sk_floats(q6k_gemm_sk_grid());
+	const size_t skf = q6k_gemm_sk_floats(m, n_out, n_in);   // the sums of a split K (workspace slot 6)
+	if (skf) {
 		void *p = nullptr;
 		if (int rc = workspace(6, skf * 4, &p)) return rc;
 		skp = (float *)p;
 	}
-	return q6k_gemm_split(y, w, xh, xl, esc, bias, m, n_out, n_in, false, skp, skf);
+	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, skp, skf);
 }
 
-// The stream-K slots of a launch on G workgroups (floats).
-size_t q6k_gemm_sk_floats(int G) { return (size_t)G * 2 * 512 * 16; }
-int q6k_gemm_sk_grid() { return cu_count() / kXcds * kXcds; }
+namespace {
 
-int q6k_gemm_split(float *y, const void *w, const _Float16 *xh, const _Float16 *xl, const float *esc,
-                   const float *bias, int m, int n_out, int n_in, bool add, float *skp, size_t skp_floats) {
+// The launch of m x n_out x n_in with `cap` floats of slots: the 64- or 128-row
+// tiles (tm = 0), or tm tokens x 256 rows and the workgroups that share a tile's K (no
+// more than the CUs take at once, one workgroup per CU: registers and 80 KB of
+// LDS). Chosen by what each would take: per super-block 2.3 us (one tile per
+// CU) or 3.5 us per round of two for the 64-row tiles, 8.7 and 6.0 us for 128
+// and 64 tokens, the sums of a split K written and read at 4 TB/s, and a start
+// of 8.5 and 9 us. Within 25% of what 64 shapes measured (17 .. 512 tokens, 64
+// .. 18944 rows, 256 .. 2048 values: q6_k 4096 x 512 at 200 tokens 12.4 us in
+// small tiles and 19.2 in wide ones, 18944 x 512 at 200 tokens 32.4 and 27.0).
+struct Q6Plan {
+	int tm, tiles, ks;
+};
+Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, size_t cap) {
+	const int NB = n_in / kQK, cus = cu_count();
+	Q6Plan best{};
+	const int small = ((m + kTM - 1) / kTM) * ((n_out + kTN - 1) / kTN);
+	double best_us = 8.5 + NB * (small <= cus ? 2.3 : 3.5 * ((small + 2 * cus - 1) / (2 * cus)));
+	if (g_q6_gemm_tm > 0) best_us = 1e30;
+	for (int tm = 128; tm >= 64; tm -= 64) {
+		if (g_q6_gemm_tm > 0 && tm != g_q6_gemm_tm) continue;
+		Q6Plan p;
+		p.tm = tm;
+		p.tiles = ((m + tm - 1) / tm) * ((n_out + kQ6TN - 1) / kQ6TN);
+		const int most = !g_q6_gemm_sk || cus < 2 * p.tiles ? 1 : cus / p.tiles < NB ? cus / p.tiles : NB;
+		for (p.ks = 1; p.ks <= most; p.ks++) {
+			const size_t slots = (size_t)p.tiles * p.ks * q6w_slot(tm);
+			if (p.ks > 1 && slots > cap) break;
+			const int rounds = p.ks > 1 ? 1 : (p.tiles + cus - 1) / cus;
+			const double us = 9.0 + rounds * ((NB + p.ks - 1) / p.ks) * (tm == 128 ? 8.7 : 6.0) +
+			                  (p.ks > 1 ? 4.0 + (double)slots * 8 / 4e6 : 0.0);
+			if (us < best_us) {
+				best = p;
+				best_us = us;
+			}
+		}
+	}
+	return best;
+}
+
+}  // namespace
+
+size_t q6k_gemm_sk_floats(int m, int n_out, int n_in) {
+	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, ~(size_t)0);
+	return p.tm && p.ks > 1 ? (size_t)p.tiles * p.ks * q6w_slot(p.tm) : 0;
+}
+// (tiles * ks <= the CUs when ks > 1)
+size_t q6k_gemm_sk_max_floats() { return (size_t)cu_count() * q6w_slot(128); }
+
+int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, const float *bias, int m, int n_out,
+               int n_in, bool add, float *skp, size_t skp_floats) {
 	if (int rc = check_gemm("Q6_K GEMM", m, n_out, n_in, (size_t)n_in / kQK * kQ6Bytes, w)) return rc;
-	if (m <= kSkMaxTokens) return set_error(HAKO_GPU_EINVAL, "Q6_K GEMM on split rows needs m > %d", kSkMaxTokens);
-	// 128-row tiles when they still give about one workgroup per CU
-	const int wide_tiles = ((m + kTM - 1) / kTM) * ((n_out + 127) / 128);
-	const bool wide = g_q6_gemm_tn == 128 || (g_q6_gemm_tn < 0 && 4 * wide_tiles >= 3 * cu_count());
-	const int tn = wide ? 128 : kTN;
-	const int gm = gemm_gm(m, n_out, (double)kTM * n_in * 4, (double)tn * (n_in / kQK) * kQ6Bytes, tn);
-	// stream-K when the 128-row tiles leave CUs idle and the caller holds the slots
-	const int G = q6k_gemm_sk_grid();
-	const bool sk = wide && g_q6_gemm_sk && skp && skp_floats >= q6k_gemm_sk_floats(G) && wide_tiles < G &&
-	                n_in / kQK >= 2;
-	if (sk) {
-		hipLaunchKernelGGL((q6k_gemm_kernel<128, true, true>), dim3(G), dim3(4 * 128), 2 * q6g_buf_bytes(128), stream(),
-		                   (const uint8_t *)w, xh, xl, esc, bias, y, m, n_out, n_in, add ? 1 : 0, gm, skp);
+	if (m <= kSkMaxTokens) return set_error(HAKO_GPU_EINVAL, "Q6_K GEMM tiles need m > %d", kSkMaxTokens);
+	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, skp ? skp_floats : 0);
+	if (!p.tm) {
+		_Float16 *xh = (_Float16 *)act, *xl = xh + (size_t)m * n_in;
+		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
+		// 128-row tiles when they still give about one workgroup per CU
+		const bool wide = 4 * (((m + kTM - 1) / kTM) * ((n_out + 127) / 128)) >= 3 * cu_count();
+		const int tn = wide ? 128 : kTN;
+		const int gm = gemm_gm(m, n_out, (double)kTM * n_in * 4, (double)tn * (n_in / kQK) * kQ6Bytes, tn);
+		if (wide)
+			hipLaunchKernelGGL((q6k_gemm_kernel<128, true>), dim3(gemm_grid(m, n_out, 128)), dim3(4 * 128),
+			                   2 * q6g_buf_bytes(128), stream(), (const uint8_t *)w, xh, xl, esc, bias, y, m, n_out, n_in,
+			                   add ? 1 : 0, gm);
+		else
+			hipLaunchKernelGGL((q6k_gemm_kernel<kTN, false>), dim3(gemm_grid(m, n_out)), dim3(4 * kTN), q6g_buf_bytes(kTN),
+			                   stream(), (const uint8_t *)w, xh, xl, esc, bias, y, m, n_out, n_in, add ? 1 : 0, gm);
 		HK_LAUNCHED("q6k_gemm");
-		hipLaunchKernelGGL(q6k_gemm_sk_fixup_kernel, dim3(wide_tiles), dim3(512), 0, stream(), skp, esc, bias, y, m,
-		                   n_out, n_in / kQK, G, gm, add ? 1 : 0);
-		HK_LAUNCHED("q6k_gemm_sk_fixup");
 		return ok();
 	}
-	if (wide)
-		hipLaunchKernelGGL((q6k_gemm_kernel<128, true>), dim3(gemm_grid(m, n_out, 128)), dim3(4 * 128),
-		                   2 * q6g_buf_bytes(128), stream(), (const uint8_t *)w, xh, xl, esc, bias, y, m, n_out, n_in,
-		                   add ? 1 : 0, gm, nullptr);
-	else
-		hipLaunchKernelGGL((q6k_gemm_kernel<kTN, false>), dim3(gemm_grid(m, n_out)), dim3(4 * kTN), q6g_buf_bytes(kTN),
-		                   stream(), (const uint8_t *)w, xh, xl, esc, bias, y, m, n_out, n_in, add ? 1 : 0, gm, nullptr);
-	HK_LAUNCHED("q6k_gemm");
-	return ok();
+	uint8_t *xp = (uint8_t *)act;
+	if (n_in <= 1024) {
+		hipLaunchKernelGGL((f16_pack8_kernel<256, 4>), dim3((m + 7) / 8), dim3(256), 0, stream(), x, esc, xp, m, n_in);
+		HK_LAUNCHED("f16_pack8");
+	} else if (n_in <= kPackK) {
+		hipLaunchKernelGGL((f16_pack8_kernel<kEscT, kPackK / kEscT>), dim3((m + 7) / 8), dim3(kEscT), 0, stream(), x, esc, xp, m,
+		                   n_in);
+		HK_LAUNCHED("f16_pack8");
+	} else {
+		hipLaunchKernelGGL(f16_esc_kernel, dim3(m), dim3(kEscT), 0, stream(), x, esc, n_in);
+		HK_LAUNCHED("f16_esc");
+		hipLaunchKernelGGL(f16_pack_kernel, dim3((m + 31) / 32, n_in / kQK), dim3(256), 0, stream(), x, esc, xp, m, n_in);
+		HK_LAUNCHED("f16_pack");
+	}
+	const int gm = gemm_gm(m, n_out, (double)p.tm * n_in * 4, (double)kQ6TN * (n_in / kQK) * kQ6Bytes, kQ6TN, p.tm);
+	const dim3 grid(kXcds * ((p.tiles * p.ks + kXcds - 1) / kXcds));
+	auto launch = [&](auto tmc) -> int {
+		constexpr int TM = decltype(tmc)::value;
+		hipLaunchKernelGGL((q6k_gemm_wide_kernel<TM>), grid, dim3(kQ6T), 0, stream(), (const uint8_t *)w, xp, esc, bias, y,
+		                   m, n_out, n_in, add ? 1 : 0, gm, p.ks, skp);
+		HK_LAUNCHED("q6k_gemm");
+		if (p.ks > 1) {
+			hipLaunchKernelGGL((q6k_gemm_fix_kernel<TM>), dim3(p.tiles * (TM / 8)), dim3(kQ6T), 0, stream(), skp, esc, bias, y,
+			                   m, n_out, p.tiles, p.ks, gm, add ? 1 : 0);
+			HK_LAUNCHED("q6k_gemm_fix");
+		}
+		return ok();
+	};
+	return p.tm == 128 ? launch(std::integral_constant<int, 128>{}) : launch(std::integral_constant<int, 64>{});
 }
 
 }  // namespace hako

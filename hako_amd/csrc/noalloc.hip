@@ -122,10 +122,11 @@ extern "C" int hako_gpu_matmul_batch_noalloc(float *y, const float *x, int type,
 	_Float16 *xh = (_Float16 *)base;
 	_Float16 *xl = (_Float16 *)(base + half);
 	float *esc = (float *)(base + 2 * half);
-	if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 	if (skinny) {
+		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 		if (int rc = q6k_skinny(segs, kSkStore, xh, xl, esc, m, n_in, n_out, part, pf)) return rc;
-	} else if (int rc = q6k_gemm_split(y, w, xh, xl, esc, bias, m, n_out, n_in, false)) {
+	} else if (int rc = q6k_gemm_x(y, w, x, base, esc, bias, m, n_out, n_in, false, (float *)(base + align256(act)),
+	                             (kScratchBytes - align256(act)) / 4)) {
 		return rc;
 	}
 	return ok();

@@ -67,15 +67,14 @@ int f16_split(const float *x, _Float16 *xh, _Float16 *xl, float *esc, int m, int
 // [m][ld]): Store, Add, or SwiGLU (segment 0 gate and segment 1 up, both
 // rows [0, F) with F % 32 == 0; out of segment 0 = silu(gate)*up).
 int q4k_gemm_segs(const SkSegs &segs, int epi, const int8_t *xq, const float *xs, int m, int n_in, int vrows);
-// Q6_K x the fp16 hi/lo rows of f16_split: y[m][n_out] = (or += when add)
-// W x (+ bias).
-// skp: stream-K slots of q6k_gemm_sk_floats(q6k_gemm_sk_grid()) floats, or
-// null (then no stream-K); the launch uses them only when its 128-row tiles
-// would leave CUs idle.
-int q6k_gemm_split(float *y, const void *w, const _Float16 *xh, const _Float16 *xl, const float *esc,
-                   const float *bias, int m, int n_out, int n_in, bool add, float *skp = nullptr,
-                   size_t skp_floats = 0);
-size_t q6k_gemm_sk_floats(int G);
-int q6k_gemm_sk_grid();
+// Q6_K x fp32 rows x [m][n_in] (16-byte aligned): y[m][n_out] = (or += when
+// add) W x (+ bias). act: m*n_in*4 bytes (16-byte aligned) for the fp16 hi/lo
+// operands, esc: m floats. skp: room for the sums of a split K, best
+// q6k_gemm_sk_floats(m, n_out, n_in) floats (fewer, or null: K is split less,
+// or not).
+int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, const float *bias, int m, int n_out,
+               int n_in, bool add, float *skp = nullptr, size_t skp_floats = 0);
+size_t q6k_gemm_sk_floats(int m, int n_out, int n_in);
+size_t q6k_gemm_sk_max_floats();   // of any launch
 
 }  // namespace hako

@@ -220,6 +220,32 @@ def test_q6k_gemm_stream_k(gpu, oracle, m, n_out, n_in):
         gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
 
 
+@pytest.mark.parametrize("m,n_out,n_in", [(17, 1, 256), (33, 257, 512), (64, 255, 1024), (65, 256, 1280),
+                                         (128, 520, 4096), (129, 300, 4352), (161, 513, 2816)])
+def test_q6k_gemm_wide_tile_edges(gpu, oracle, m, n_out, n_in):
+    """256-row tiles at the edges of their token tiles (32, 64, 128), rows, and
+    the activation layouts (rows of up to 1024, 4096 and more values), K whole
+    and split, with rows of very different magnitude. Per output, hi + lo is
+    within 2^-22 of a row's largest activation and the sums are fp32: within
+    the bar of the other GEMM tests."""
+    rng = np.random.default_rng(m + n_out + n_in)
+    w = synth.q6k_weight(rng, n_out, n_in)
+    x = rng.standard_normal((m, n_in)).astype(np.float32) * np.exp2(rng.integers(-20, 20, (m, 1))).astype(np.float32)
+    bias = 0.1 * rng.standard_normal(n_out).astype(np.float32)
+    want = oracle.matmul(Q6, w, x, n_out, n_in, bias=bias, f64=True)
+    scale = np.max(np.abs(want), axis=1, keepdims=True)
+    try:
+        for tm in (64, 128):
+            gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, tm)
+            for sk in (0, 1):
+                gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, sk)
+                got = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
+                assert np.max(np.abs(got - want) / scale) < TOL
+    finally:
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
+
+
 def test_q6k_gemm_full_7b_shape_sampled_rows(gpu, oracle):
     rng = np.random.default_rng(78)
     m, n_out, n_in = 512, 3584, 18944
