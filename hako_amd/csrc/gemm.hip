@@ -293,6 +293,13 @@ __global__ __launch_bounds__(kGT, 3) void q4k_gemm_kernel(const SkSegs segs, con
 // segment: segment starts are multiples of 64); SwiGLU features
 // 16u .. 16u+15, MFMA rows 0-15 their gate rows and 16-31 their up rows, so a
 // lane holds each feature's gate and up sums side by side.
+// With few units per workgroup (a short prompt, a small matrix) most waves
+// would have none, and the others a serial chain over the whole K: KW lets kw
+// waves share a unit, a range of K each, their sums meeting in LDS in order of
+// K. 2048 x 2048 at 77 tokens (one unit per workgroup, 8 waves each) 17.2 ->
+// 12.5 us, 2048 x 3584 at 200 tokens (three) 26.0 -> 19.2; from four units on
+// only where K is long (2048 x 1024 at 512 tokens 15.5 -> 16.3, x 3584 30.6 ->
+// 28.5). One wave per unit is its own instance: the two in one spill registers.
 // Grid: token tiles x R row ranges, in XCD-contiguous order with the token
 // tiles minor: the workgroups of one XCD share a row range, whose weights
 // then come from that XCD's L2 after the first read.
@@ -302,11 +309,11 @@ constexpr int kRMaxK = 3840;     // largest K whose token tile fits 160 KB of LD
 
 __host__ __device__ inline size_t q4k_res_lds(int K) { return (size_t)kRT * (K + 16) + (size_t)(K / 32) * kRT * 8; }
 
-template <int EPI>
+template <int EPI, bool KW>
 __global__ __launch_bounds__(kRWaves * kWave, 1) void q4k_gemm_res_kernel(const SkSegs segs,
                                                                        const int8_t *__restrict__ xq,
                                                                        const float *__restrict__ xs, int M, int K,
-                                                                       int R, int units) {
+                                                                       int R, int units, int kw) {
 	extern __shared__ __align__(16) uint8_t res_lds[];
 	const int AP = K + 16;                              // bytes per staged token row
 	int8_t *a_s = (int8_t *)res_lds;
@@ -371,9 +378,12 @@ __global__ __launch_bounds__(kRWaves * kWave, 1) void q4k_gemm_res_kernel(const 
 		uint4 q[4];   // qs bytes 32g + 16kh .. +16 of the lane's row
 		uint4 h;      // d, dmin, 12 scale bytes
 	};
-	for (int u = u0 + wave; u < u1; u += kRWaves) {
+	const int slot = KW ? wave / kw : wave, part = KW ? wave - slot * kw : 0;
+	for (int u = u0 + slot; KW || u < u1; u += kRWaves) {   // (KW: once, every wave)
 		// the lane's weight row (clamped into its matrix; rows past the end are
 		// computed and not stored)
+		const bool has = !KW || (u < u1 && slot < kRWaves / kw);   // a wave past the units has no super-blocks
+		const int kb0 = KW && has ? part * NB / kw : 0, kb1 = !KW ? NB : has ? (part + 1) * NB / kw : 0;
 		const int r32 = 32 * u;
 		const int si = EPI == kSkSwiGLU ? 0
 		               : (segs.n > 2 && r32 >= segs.s[2].row0) ? 2 : (segs.n > 1 && r32 >= segs.s[1].row0) ? 1 : 0;
@@ -434,17 +444,32 @@ __global__ __launch_bounds__(kRWaves * kWave, 1) void q4k_gemm_res_kernel(const 
 		// it), so the wait before each block's arithmetic counts only the older
 		// set
 		Wt wa, wb;
-		load(wa, 0);
-		int kb = 0;
-		for (; kb + 1 < NB; kb += 2) {
+		load(wa, kb0);
+		int kb = kb0;
+		for (; kb + 1 < kb1; kb += 2) {
 			load(wb, kb + 1);
 			__builtin_amdgcn_sched_barrier(0);   // issued here, not next to their use
 			compute(wa, kb);
-			load(wa, min(kb + 2, NB - 1));
+			load(wa, min(kb + 2, kb1 - 1));
 			__builtin_amdgcn_sched_barrier(0);
 			compute(wb, kb + 1);
 		}
-		if (kb < NB) compute(wa, kb);   // odd NB: the last block, loaded into wa
+		if (kb < kb1) compute(wa, kb);   // odd count: the last block, loaded into wa
+		if constexpr (KW) {
+			// the parts of a unit meet in LDS (the token tile's place), added in order of K
+			float *red = (float *)res_lds + lane;
+			__syncthreads();
+#pragma unroll
+			for (int v = 0; v < 16; v++) red[(wave * 16 + v) * kWave] = acc[v] + accm[v];
+			__syncthreads();
+			if (part || !has) return;
+#pragma unroll
+			for (int v = 0; v < 16; v++) acc[v] = red[(wave * 16 + v) * kWave];
+			for (int q = 1; q < kw; q++)
+#pragma unroll
+				for (int v = 0; v < 16; v++) acc[v] += red[((wave + q) * 16 + v) * kWave];
+			accm = v16f{};
+		}
 
 		// 3. epilogue; lane: token m0 + li, MFMA rows 8q4 + 4kh + r
 		const int tok = m0 + li;
@@ -461,6 +486,7 @@ __global__ __launch_bounds__(kRWaves * kWave, 1) void q4k_gemm_res_kernel(const 
 							            (acc[4 * q4 + 8 + r] + accm[4 * q4 + 8 + r]);
 				}
 			}
+			if (KW) return;
 			continue;
 		}
 		const int ld = __builtin_amdgcn_readfirstlane(S.ld);
@@ -484,6 +510,7 @@ __global__ __launch_bounds__(kRWaves * kWave, 1) void q4k_gemm_res_kernel(const 
 #pragma unroll
 		for (int v = 0; v < 16; v++)
 			st_f32(ors, off[v], EPI == kSkAdd ? ev[v] + (acc[v] + accm[v]) : (acc[v] + accm[v]) + ev[v]);
+		if (KW) return;
 	}
 }
 
@@ -1273,11 +1300,22 @@ int q4k_gemm_segs(const SkSegs &segs, int epi, const int8_t *xq, const float *xs
 		const int units = epi == kSkSwiGLU ? (segs.s[0].rows + 15) / 16 : (vrows + 31) / 32;
 		const int G = mt * R;
 		const dim3 rgrid(kXcds * ((G + kXcds - 1) / kXcds)), rblock(kRWaves * kWave);
-		const size_t lds = q4k_res_lds(n_in);
+		// kw waves share a unit where a workgroup has few (see the kernel)
+		const int upw = (units + R - 1) / R, NB = n_in / kQK;
+		const int kw = upw > 4 || (upw > 2 && NB <= 2 * upw) ? 1 : kRWaves / upw < NB ? kRWaves / upw : NB;
+		const size_t tile_lds = q4k_res_lds(n_in), red_lds = kw > 1 ? (size_t)kRWaves * kWave * 16 * 4 : 0;
+		const size_t lds = tile_lds > red_lds ? tile_lds : red_lds;
+		auto launch = [&](auto e) {
+			constexpr int EPI = decltype(e)::value;
+			if (kw > 1)
+				hipLaunchKernelGGL((q4k_gemm_res_kernel<EPI, true>), rgrid, rblock, lds, stream(), segs, xq, xs, m, n_in, R, units, kw);
+			else
+				hipLaunchKernelGGL((q4k_gemm_res_kernel<EPI, false>), rgrid, rblock, lds, stream(), segs, xq, xs, m, n_in, R, units, 1);
+		};
 		switch (epi) {
-		case kSkStore: hipLaunchKernelGGL(q4k_gemm_res_kernel<kSkStore>, rgrid, rblock, lds, stream(), segs, xq, xs, m, n_in, R, units); break;
-		case kSkAdd: hipLaunchKernelGGL(q4k_gemm_res_kernel<kSkAdd>, rgrid, rblock, lds, stream(), segs, xq, xs, m, n_in, R, units); break;
-		case kSkSwiGLU: hipLaunchKernelGGL(q4k_gemm_res_kernel<kSkSwiGLU>, rgrid, rblock, lds, stream(), segs, xq, xs, m, n_in, R, units); break;
+		case kSkStore: launch(std::integral_constant<int, kSkStore>{}); break;
+		case kSkAdd: launch(std::integral_constant<int, kSkAdd>{}); break;
+		case kSkSwiGLU: launch(std::integral_constant<int, kSkSwiGLU>{}); break;
 		default: return set_error(HAKO_GPU_EINVAL, "Q4_K GEMM epilogue %d", epi);
 		}
 		HK_LAUNCHED("q4k_gemm_res");

@@ -220,6 +220,33 @@ def test_q6k_gemm_stream_k(gpu, oracle, m, n_out, n_in):
         gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
 
 
+@pytest.mark.parametrize("m,n_out,n_in", [(17, 1, 512), (32, 33, 768), (33, 65, 2048), (77, 2048, 2048),
+                                         (77, 4608, 1280), (200, 3000, 3584), (512, 2048, 3840), (512, 2048, 2048)])
+def test_q4k_gemm_shared_units(gpu, oracle, m, n_out, n_in):
+    """Few 32-row units per workgroup, so that several waves share one (from
+    two waves of one super-block each to twelve, and fewer super-blocks than
+    waves); the last shape is the first past the rule. Integer inputs with one
+    (s, m) = (1, 0) per block and unit scales: every output is exact in
+    fp32 whatever the order of the sums."""
+    rng = np.random.default_rng(m + n_out + n_in)
+    nb = n_in // 256
+    w = synth.q4k_weight(rng, n_out, n_in).reshape(n_out * nb, 144).copy()
+    w[:, 0:4] = np.frombuffer(np.float16([1.0, 1.0]).tobytes(), np.uint8)
+    w[:, 4:16] = _one_hot_scales(n_out * nb, 5, "s")
+    w = w.reshape(n_out, nb * 144)
+    xq = rng.integers(-127, 128, (m, n_in)).astype(np.int8)
+    got = run_q4k_gemm(gpu, w, xq, np.ones((m, n_in // 32), np.float32), n_out, n_in)
+    q = (w.reshape(n_out, nb, 144)[:, :, 16 + 64:16 + 96] >> 4).astype(np.float64)   # sub-block 5: high nibbles
+    want = xq.reshape(m, nb, 8, 32)[:, :, 5].reshape(m, -1).astype(np.float64) @ q.reshape(n_out, -1).T
+    assert np.array_equal(got, want.astype(np.float32))
+    if m * n_out * n_in < 1 << 29:   # and random inputs against the oracle
+        w = synth.q4k_weight(rng, n_out, n_in)
+        x = rng.standard_normal((m, n_in)).astype(np.float32)
+        bias = 0.1 * rng.standard_normal(n_out).astype(np.float32)
+        got = run_batch(gpu, Q4, w, x, n_out, n_in, bias)
+        assert maxabs_rel(got, oracle.matmul(Q4, w, x, n_out, n_in, bias=bias, f64=True)) < TOL
+
+
 @pytest.mark.parametrize("m,n_out,n_in", [(17, 1, 256), (33, 257, 512), (64, 255, 1024), (65, 256, 1280),
                                          (128, 520, 4096), (129, 300, 4352), (161, 513, 2816)])
 def test_q6k_gemm_wide_tile_edges(gpu, oracle, m, n_out, n_in):
