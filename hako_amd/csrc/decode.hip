@@ -1509,18 +1509,20 @@ int dalloc(hako_gpu_decoder *d, size_t bytes, void **p) {
 	return HAKO_GPU_OK;
 }
 
-// The decoder's pinned slots, for results of up to `bytes`.
-int stage_alloc(hako_gpu_decoder *d, size_t bytes) {
+// The decoder's pinned slots, for results of up to `bytes`. Without them (no
+// pinned memory to be had) results are copied directly.
+void stage_alloc(hako_gpu_decoder *d, size_t bytes) {
 	const size_t n = (bytes + kStageSlot - 1) / kStageSlot, slots = n < (size_t)kStageSlots ? n : kStageSlots;
 	d->stage_slot = n > 1 ? kStageSlot : (bytes + 255) & ~(size_t)255;
-	if (hipHostMalloc((void **)&d->stage, slots * d->stage_slot, hipHostMallocDefault) != hipSuccess) {
-		(void)hipGetLastError();
-		d->stage = nullptr;
-		return set_error(HAKO_GPU_ENOMEM, "decoder allocation of %zu pinned bytes", slots * d->stage_slot);
-	}
 	d->stage_slots = (int)slots;
-	for (hipEvent_t &e : d->stage_ev) HK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-	return HAKO_GPU_OK;
+	bool ok = hipHostMalloc((void **)&d->stage, slots * d->stage_slot, hipHostMallocDefault) == hipSuccess;
+	if (!ok) d->stage = nullptr;
+	for (size_t i = 0; ok && i < slots; i++) ok = hipEventCreateWithFlags(&d->stage_ev[i], hipEventDisableTiming) == hipSuccess;
+	if (!ok) {
+		(void)hipGetLastError();
+		if (d->stage) (void)hipHostFree(d->stage);
+		d->stage = nullptr;
+	}
 }
 
 // dst (host) = bytes of src (device), after everything on the stream. Ordinary
@@ -1533,7 +1535,7 @@ int read_back(hako_gpu_decoder *d, void *dst, const void *src, size_t bytes) {
 	hipPointerAttribute_t at{};
 	const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
 	if (!known) (void)hipGetLastError();
-	if (known || bytes <= 16384) {
+	if (known || bytes <= 16384 || !d->stage) {
 		HK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream()));
 		HK_HIP(hipStreamSynchronize(stream()));
 		return HAKO_GPU_OK;
@@ -2350,7 +2352,6 @@ int hako_gpu_decoder_create(const hako_gpu_model *m, int n_seq, int max_seq, hak
 		d->skpart_floats = skpart;
 	}
 #undef HK_ALLOC
-	if (!rc) rc = stage_alloc(d, sizeof(float) * n_seq * m->vocab);
 	if (rc) {
 		hako_gpu_decoder_destroy(d);
 		return rc;
@@ -2374,6 +2375,8 @@ int hako_gpu_decoder_create(const hako_gpu_model *m, int n_seq, int max_seq, hak
 		hako_gpu_decoder_destroy(d);
 		return hip_fail(e, "decoder init", __FILE__, __LINE__);
 	}
+	const size_t logit_bytes = sizeof(float) * n_seq * m->vocab, ring_bytes = sizeof(int) * n_seq * max_seq;
+	stage_alloc(d, logit_bytes > ring_bytes ? logit_bytes : ring_bytes);
 	*out = d;
 	return ok();
 }
