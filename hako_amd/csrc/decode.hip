@@ -1482,7 +1482,6 @@ struct hako_gpu_decoder {
 	float *pf_xs = nullptr, *pf_esc = nullptr;  // fp16 hi/lo operands of the SwiGLU rows (chunk*ffn*4 bytes), esc[chunk]
 	uint8_t *pf_xh = nullptr;
 	float *pf_sk = nullptr;   // sums of the down matmul's split K
-	size_t pf_sk_floats = 0;
 	int *pf_tok = nullptr, *pf_pos = nullptr;
 	int pf_chunk = 0;   // most tokens per prefill pass
 	size_t pf_part_bytes = 0;   // capacity of pf_part
@@ -2141,8 +2140,7 @@ int prefill_alloc(hako_gpu_decoder *d) {
 	HK_ALLOC(d->pf_xs, 4 * C * (D > F ? D : F) / 32);
 	HK_ALLOC(d->pf_xh, 4 * C * F);
 	HK_ALLOC(d->pf_esc, 4 * C);
-	d->pf_sk_floats = q6k_gemm_sk_max_floats();
-	HK_ALLOC(d->pf_sk, 4 * d->pf_sk_floats);
+	HK_ALLOC(d->pf_sk, 4 * kQ6SplitFloats);
 	HK_ALLOC(d->pf_tok, 4 * C);
 	HK_ALLOC(d->pf_pos, 4 * C);
 #undef HK_ALLOC
@@ -2253,8 +2251,7 @@ int prefill_chunk(hako_gpu_decoder *d, int seq, const int *tokens, int n, int po
 		}
 		// down + residual: h = pf_g
 		if (n > kSkMaxTokens && B.t_down == HAKO_TYPE_Q6_K) {
-			if (int rc = q6k_gemm_x(d->pf_x, B.down, d->pf_g, d->pf_xh, d->pf_esc, nullptr, n, D, F, true, d->pf_sk,
-			                        d->pf_sk_floats))
+			if (int rc = q6k_gemm_x(d->pf_x, B.down, d->pf_g, d->pf_xh, d->pf_esc, nullptr, n, D, F, true, d->pf_sk))
 				return rc;
 		} else if (n > kSkMaxTokens && B.t_down == HAKO_TYPE_Q4_K) {
 			if (int rc = hako_gpu_quantize_q8_32(d->pf_g, n, F, d->pf_xq, d->pf_xs)) return rc;

@@ -1367,15 +1367,17 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 		if (int rc = workspace(6, skf * 4, &p)) return rc;
 		skp = (float *)p;
 	}
-	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, skp, skf);
+	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, skp);
 }
 
 namespace {
 
-// The launch of m x n_out x n_in with `cap` floats of slots: the 64- or 128-row
-// tiles (tm = 0), or tm tokens x 256 rows and the workgroups that share a tile's K (no
-// more than the CUs take at once, one workgroup per CU: registers and 80 KB of
-// LDS). Chosen by what each would take: per super-block 2.3 us (one tile per
+// The launch of m x n_out x n_in, with room for the sums of a split K or
+// without: the 64- or 128-row tiles (tm = 0), or tm tokens x 256 rows and the
+// workgroups that share a tile's K (no more than the CUs take at once, one
+// workgroup per CU: registers and 80 KB of LDS; and no more sums than
+// kQ6SplitFloats, which every caller's room holds, so that all of them split
+// alike and give the same bits). Chosen by what each would take: per super-block 2.3 us (one tile per
 // CU) or 3.5 us per round of two for the 64-row tiles, 8.7 and 6.0 us for 128
 // and 64 tokens, the sums of a split K written and read at 4 TB/s, and a start
 // of 8.5 and 9 us. Within 25% of what 64 shapes measured (17 .. 512 tokens, 64
@@ -1384,7 +1386,7 @@ namespace {
 struct Q6Plan {
 	int tm, tiles, ks;
 };
-Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, size_t cap) {
+Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, bool room) {
 	const int NB = n_in / kQK, cus = cu_count();
 	Q6Plan best{};
 	const int small = ((m + kTM - 1) / kTM) * ((n_out + kTN - 1) / kTN);
@@ -1395,10 +1397,10 @@ Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, size_t cap) {
 		Q6Plan p;
 		p.tm = tm;
 		p.tiles = ((m + tm - 1) / tm) * ((n_out + kQ6TN - 1) / kQ6TN);
-		const int most = !g_q6_gemm_sk || cus < 2 * p.tiles ? 1 : cus / p.tiles < NB ? cus / p.tiles : NB;
+		const int most = !room || !g_q6_gemm_sk || cus < 2 * p.tiles ? 1 : cus / p.tiles < NB ? cus / p.tiles : NB;
 		for (p.ks = 1; p.ks <= most; p.ks++) {
 			const size_t slots = (size_t)p.tiles * p.ks * q6w_slot(tm);
-			if (p.ks > 1 && slots > cap) break;
+			if (p.ks > 1 && slots > kQ6SplitFloats) break;
 			const int rounds = p.ks > 1 ? 1 : (p.tiles + cus - 1) / cus;
 			const double us = 9.0 + rounds * ((NB + p.ks - 1) / p.ks) * (tm == 128 ? 8.7 : 6.0) +
 			                  (p.ks > 1 ? 4.0 + (double)slots * 8 / 4e6 : 0.0);
@@ -1414,17 +1416,15 @@ Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, size_t cap) {
 }  // namespace
 
 size_t q6k_gemm_sk_floats(int m, int n_out, int n_in) {
-	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, ~(size_t)0);
+	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, true);
 	return p.tm && p.ks > 1 ? (size_t)p.tiles * p.ks * q6w_slot(p.tm) : 0;
 }
-// (tiles * ks <= the CUs when ks > 1)
-size_t q6k_gemm_sk_max_floats() { return (size_t)cu_count() * q6w_slot(128); }
 
 int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, const float *bias, int m, int n_out,
-               int n_in, bool add, float *skp, size_t skp_floats) {
+               int n_in, bool add, float *skp) {
 	if (int rc = check_gemm("Q6_K GEMM", m, n_out, n_in, (size_t)n_in / kQK * kQ6Bytes, w)) return rc;
 	if (m <= kSkMaxTokens) return set_error(HAKO_GPU_EINVAL, "Q6_K GEMM tiles need m > %d", kSkMaxTokens);
-	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, skp ? skp_floats : 0);
+	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, skp != nullptr);
 	if (!p.tm) {
 		_Float16 *xh = (_Float16 *)act, *xl = xh + (size_t)m * n_in;
 		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;

@@ -4,8 +4,9 @@
 // hipMalloc).
 //
 // Its scratch (the q8_32 rows and scales of a Q4_K activation, the fp16 hi/lo
-// rows of a Q6_K activation, the split-K partial sums of a skinny launch)
-// lives in one file-scope device array of kScratchBytes. Each device the
+// operands of a Q6_K activation, the split-K partial sums of a skinny launch,
+// the sums of a larger Q6_K matmul's split K) lives in one file-scope device
+// array. Each device the
 // library runs on holds its own copy of the array at its own address until
 // the process ends; hako_gpu_init looks that address up once per device
 // (noalloc_setup) and every call passes it, never the array's name, to the
@@ -26,11 +27,14 @@ namespace hako {
 namespace {
 
 // 7B-prompt shapes fit: 512 tokens x 18944 inputs as fp16 hi + lo (38.8 MB),
-// or as q8_32 rows (10.9 MB), plus the partials of a 16-token split.
+// or as q8_32 rows (10.9 MB), plus the partials of a 16-token split. Behind
+// them, the sums of a split K: room for any launch, so that a matmul splits K
+// here as hako_gpu_matmul_batch does, whatever its activation takes.
 constexpr size_t kScratchBytes = (size_t)48 << 20;
+constexpr size_t kSplitBytes = kQ6SplitFloats * 4;
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) uint8_t scratch[kScratchBytes];
+static __device__ __align__(256) uint8_t scratch[kScratchBytes + kSplitBytes];
 
 std::mutex g_mu;
 void *g_scratch[kMaxDevices];   // device address of `scratch`, per device
@@ -125,8 +129,7 @@ extern "C" int hako_gpu_matmul_batch_noalloc(float *y, const float *x, int type,
 	if (skinny) {
 		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 		if (int rc = q6k_skinny(segs, kSkStore, xh, xl, esc, m, n_in, n_out, part, pf)) return rc;
-	} else if (int rc = q6k_gemm_x(y, w, x, base, esc, bias, m, n_out, n_in, false, (float *)(base + align256(act)),
-	                             (kScratchBytes - align256(act)) / 4)) {
+	} else if (int rc = q6k_gemm_x(y, w, x, base, esc, bias, m, n_out, n_in, false, (float *)(base + kScratchBytes))) {
 		return rc;
 	}
 	return ok();

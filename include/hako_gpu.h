@@ -208,10 +208,11 @@ int hako_gpu_matmul_batch(float *y, const float *x, int type, const void *w,
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, kernels and results (bit for bit) as hako_gpu_matmul_batch;
- * its scratch (activation rows in q8_32 or fp16 hi/lo form, split-K partials)
- * is a 48 MiB array that each device holds until the process ends, enough
- * for 512 tokens x 18944 inputs of either type. A call that needs more is
- * refused with HAKO_GPU_EINVAL and a message. Calls on one device share the
+ * its scratch is an 80 MiB array that each device holds until the process
+ * ends: 48 MiB for the activation rows in q8_32 or fp16 hi/lo form (and the
+ * partials of up to 16 tokens), enough for 512 tokens x 18944 inputs of either
+ * type, and 32 MiB for the sums of a split K. A call whose rows need more
+ * than their 48 MiB is refused with HAKO_GPU_EINVAL and a message. Calls on one device share the
  * array: calls that overlap in time on one device (several streams, or
  * graphs replayed concurrently) race. */
 int hako_gpu_matmul_batch_noalloc(float *y, const float *x, int type, const void *w,
