@@ -1346,6 +1346,11 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 	const size_t half_bytes = (size_t)m * n_in * 2, esc_off = 2 * ((half_bytes + 255) & ~(size_t)255);
 	void *ws = nullptr;
 	if (int rc = workspace(3, esc_off + (size_t)m * 4, &ws)) return rc;
+	// and the sums of a split K, room for any launch with the first call of all: a
+	// call whose rows fit workspace 3 can then be captured whatever it splits.
+	// Where there is no memory for it, K stays whole.
+	void *skp = nullptr;
+	if (workspace(6, kQ6SplitFloats * 4, &skp)) skp = nullptr;
 	float *esc = (float *)((uint8_t *)ws + esc_off);
 	if (m <= kSkMaxTokens) {   // a few tokens: the skinny kernel
 		_Float16 *xh = (_Float16 *)ws;
@@ -1360,14 +1365,7 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 		if (int rc = q6k_skinny(segs, kSkStore, xh, xl, esc, m, n_in, n_out, part, pf)) return rc;
 		return ok();
 	}
-	float *skp = nullptr;
-	const size_t skf = q6k_gemm_sk_floats(m, n_out, n_in);   // the sums of a split K (workspace slot 6)
-	if (skf) {
-		void *p = nullptr;
-		if (int rc = workspace(6, skf * 4, &p)) return rc;
-		skp = (float *)p;
-	}
-	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, skp);
+	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, (float *)skp);
 }
 
 namespace {
@@ -1414,11 +1412,6 @@ Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, bool room) {
 }
 
 }  // namespace
-
-size_t q6k_gemm_sk_floats(int m, int n_out, int n_in) {
-	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, true);
-	return p.tm && p.ks > 1 ? (size_t)p.tiles * p.ks * q6w_slot(p.tm) : 0;
-}
 
 int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, const float *bias, int m, int n_out,
                int n_in, bool add, float *skp) {

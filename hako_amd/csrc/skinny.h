@@ -69,11 +69,10 @@ int f16_split(const float *x, _Float16 *xh, _Float16 *xl, float *esc, int m, int
 int q4k_gemm_segs(const SkSegs &segs, int epi, const int8_t *xq, const float *xs, int m, int n_in, int vrows);
 // Q6_K x fp32 rows x [m][n_in] (16-byte aligned): y[m][n_out] = (or += when
 // add) W x (+ bias). act: m*n_in*4 bytes (16-byte aligned) for the fp16 hi/lo
-// operands, esc: m floats. skp: room for the sums of a split K,
-// q6k_gemm_sk_floats(m, n_out, n_in) floats (null: K stays whole).
+// operands, esc: m floats. skp: kQ6SplitFloats floats for the sums of a split K
+// (null: K stays whole).
 int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, const float *bias, int m, int n_out,
                int n_in, bool add, float *skp);
-size_t q6k_gemm_sk_floats(int m, int n_out, int n_in);
 constexpr size_t kQ6SplitFloats = (size_t)256 * 128 * 256;   // of any launch: 256 workgroups of 128 x 256 sums
 
 }  // namespace hako

@@ -295,3 +295,49 @@ def test_gemm_bad_shapes_are_rejected(gpu):
         gpu.matmul_batch(dy, dx, Q6, dw, None, 0, 4, 256)
     for b in (dw, dx, dy):
         b.free()
+
+
+_CAPTURED = """
+import sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+from hako_amd import synth
+from hako_amd.gpu import Gpu
+gpu, rng = Gpu(0), np.random.default_rng(4)
+wm, wk, m, n_out, n_in = int(sys.argv[2]), int(sys.argv[3]), 32, 256, 4096
+
+def operands(m, n_out, n_in):
+    x = rng.standard_normal((m, n_in)).astype(np.float32)
+    return gpu.alloc(4 * m * n_out), gpu.upload(x), synth.TYPE_Q6_K, gpu.upload(synth.q6k_weight(rng, n_out, n_in)), None, m, n_out, n_in
+
+first, call = operands(wm, 64, wk), operands(m, n_out, n_in)
+gpu.matmul_batch(*first)
+gpu.sync()
+gpu.capture_begin()
+gpu.matmul_batch(*call)
+graph = gpu.capture_end()
+eager = gpu.alloc(4 * m * n_out)
+for _ in range(3):
+    gpu.h2d(call[0], np.zeros((m, n_out), np.float32))
+    gpu.graph_launch(graph)
+    got = gpu.download(call[0], np.float32, (m, n_out))
+    gpu.matmul_batch(eager, *call[1:])
+    want = gpu.download(eager, np.float32, (m, n_out))
+    assert np.any(want) and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    print("replayed", flush=True)
+"""
+
+
+@pytest.mark.parametrize("wm,wk", [(512, 256), (16, 18944)])
+def test_q6k_gemm_is_captured_after_another_shape(wm, wk):
+    """A Q6_K matmul whose activation fits the workspace of an earlier call can
+    be captured, also where it splits K and the earlier call (one super-block;
+    16 tokens) did not: the room for the sums is there since the first call. In
+    a process of its own, whose workspaces hold nothing else."""
+    import os
+    import subprocess
+    import sys
+    repo = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _CAPTURED, repo, str(wm), str(wk)], capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
