@@ -1454,7 +1454,7 @@ void dec_set_attn_parts(int v) { g_dec_attn_parts = v > 0 && v <= 8 ? v : 0; }
 using namespace hako;
 
 constexpr int kStageSlots = 4;
-constexpr size_t kStageSlot = (size_t)2 << 20;   // most bytes of a slot
+constexpr size_t kStageSlot = (size_t)2 << 20;   // bytes
 
 struct hako_gpu_decoder {
 	hako_gpu_model m{};
@@ -1488,7 +1488,6 @@ struct hako_gpu_decoder {
 	std::vector<void *> allocs;
 	// pinned slots that results pass through on their way to the host (read_back)
 	uint8_t *stage = nullptr;
-	size_t stage_slot = 0;
 	int stage_slots = 0;
 	hipEvent_t stage_ev[kStageSlots] = {};
 	hipGraphExec_t exec = nullptr;
@@ -1508,13 +1507,14 @@ int dalloc(hako_gpu_decoder *d, size_t bytes, void **p) {
 	return HAKO_GPU_OK;
 }
 
-// The decoder's pinned slots, for results of up to `bytes`. Without them (no
-// pinned memory to be had) results are copied directly.
+// The decoder's pinned slots, for results of up to `bytes`, where these pass
+// through slots at all (read_back). Without them (no pinned memory to be had)
+// results are copied directly.
 void stage_alloc(hako_gpu_decoder *d, size_t bytes) {
+	if (bytes <= kStageSlot) return;
 	const size_t n = (bytes + kStageSlot - 1) / kStageSlot, slots = n < (size_t)kStageSlots ? n : kStageSlots;
-	d->stage_slot = n > 1 ? kStageSlot : (bytes + 255) & ~(size_t)255;
 	d->stage_slots = (int)slots;
-	bool ok = hipHostMalloc((void **)&d->stage, slots * d->stage_slot, hipHostMallocDefault) == hipSuccess;
+	bool ok = hipHostMalloc((void **)&d->stage, slots * kStageSlot, hipHostMallocDefault) == hipSuccess;
 	if (!ok) d->stage = nullptr;
 	for (size_t i = 0; ok && i < slots; i++) ok = hipEventCreateWithFlags(&d->stage_ev[i], hipEventDisableTiming) == hipSuccess;
 	if (!ok) {
@@ -1524,22 +1524,27 @@ void stage_alloc(hako_gpu_decoder *d, size_t bytes) {
 	}
 }
 
-// dst (host) = bytes of src (device), after everything on the stream. Ordinary
-// host memory is reached through the pinned slots, several copies ahead of
-// the one being moved on by the CPU: the 16 x 152064 logits of a step (9.7 MB) took
-// 580 us as one copy to ordinary memory and take 408 this way (4 slots of 512 KB:
-// 465; the bus alone 180, the rest is the CPU's copy). Pinned (or device)
-// destinations, and results too small to matter, are copied to directly.
+// dst (host) = bytes of src (device), in stream order; complete once the
+// stream is (the caller waits for it). Large results reach ordinary host memory
+// through the pinned slots, several copies ahead of the one being moved on by
+// the CPU: the 16 x 152064 logits of a step (9.7 MB) took 580 us as one copy to
+// ordinary memory and take 408 this way (4 slots of 512 KB: 465; the bus alone
+// 180, the rest is the CPU's copy). Results of one slot or less have no copy to
+// run ahead and are copied to directly: 608 KB take 48 us that way and took 54
+// through a slot, 32 KB 7 us less too; 1.2 and 1.8 MB were the same either way.
+// So are pinned (or device) destinations.
 int read_back(hako_gpu_decoder *d, void *dst, const void *src, size_t bytes) {
 	hipPointerAttribute_t at{};
-	const bool known = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
-	if (!known) (void)hipGetLastError();
-	if (known || bytes <= 16384 || !d->stage) {
+	bool direct = bytes <= kStageSlot || !d->stage;
+	if (!direct) {
+		direct = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
+		if (!direct) (void)hipGetLastError();
+	}
+	if (direct) {
 		HK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream()));
-		HK_HIP(hipStreamSynchronize(stream()));
 		return HAKO_GPU_OK;
 	}
-	const size_t slot = d->stage_slot, n = (bytes + slot - 1) / slot, slots = (size_t)d->stage_slots;
+	const size_t slot = kStageSlot, n = (bytes + slot - 1) / slot, slots = (size_t)d->stage_slots;
 	auto len = [&](size_t i) { return i + 1 < n ? slot : bytes - i * slot; };
 	auto issue = [&](size_t i) -> hipError_t {
 		const hipError_t e = hipMemcpyAsync(d->stage + i % slots * slot, (const uint8_t *)src + i * slot, len(i),
@@ -2437,6 +2442,7 @@ int hako_gpu_decoder_generate(hako_gpu_decoder *d, const int *tokens, int n, int
 	for (int i = 0; i < n; i++) HK_HIP(hipGraphLaunch(d->exec, stream()));
 	std::vector<int> ring((size_t)d->n_seq * d->max_seq);
 	if (int rc = read_back(d, ring.data(), d->ring, sizeof(int) * ring.size())) return rc;
+	HK_HIP(hipStreamSynchronize(stream()));
 	for (int i = 0; i < n; i++)
 		for (int s = 0; s < d->n_seq; s++) out[(size_t)i * d->n_seq + s] = ring[(size_t)s * d->max_seq + i];
 	return ok();

@@ -63,7 +63,10 @@ typedef struct hako_gpu_decoder hako_gpu_decoder;
  * launches, other layers one launch per matmul. Every sum of a step has a
  * fixed order or is exact (with n_seq == 1 and Q4_K output projections their
  * 256-input block sums meet in a 64-bit fixed-point accumulator on the 2^-32
- * grid), so steps are bit-reproducible. */
+ * grid), so steps are bit-reproducible. A decoder whose results (n_seq x
+ * vocab logits, or the n_seq x max_seq token ring) exceed 2 MiB also holds up to
+ * 8 MiB of pinned host memory, which they pass through on their way to ordinary
+ * host memory; where there is none to be had they are copied directly. */
 int hako_gpu_decoder_create(const hako_gpu_model *m, int n_seq, int max_seq, hako_gpu_decoder **dec);
 int hako_gpu_decoder_destroy(hako_gpu_decoder *dec);
 

@@ -1,7 +1,8 @@
-"""Results on their way from the decoder to ordinary host memory (pinned slots
-of at most 2 MB, four of them) against the same results copied straight into
-pinned memory: the same bytes. Sizes below and above one slot, and past the
-four (so that slots are used again)."""
+"""Results on their way from the decoder to ordinary host memory (past 2 MiB
+through pinned slots of 2 MiB, at most four of them) against the same results
+copied straight into pinned memory: the same bytes. Logits below one slot, of
+exactly one and of a few bytes more, and past the four (so that slots are used
+again); a token ring past one slot."""
 import ctypes as C
 
 import numpy as np
@@ -13,15 +14,15 @@ from hako_amd.decoder import Decoder
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n_seq,vocab", [(1, 1000), (1, 150001), (4, 150001), (16, 150001)])
-def test_logits_and_tokens_reach_ordinary_memory(gpu, tmp_path, n_seq, vocab):
+@pytest.mark.parametrize("n_seq,vocab,max_seq", [(1, 1000, 16384), (1, 150001, 64), (2, 262144, 64), (2, 262145, 64),
+                                                 (4, 150001, 64), (16, 150001, 64), (16, 1000, 40000)])
+def test_logits_and_tokens_reach_ordinary_memory(gpu, tmp_path, n_seq, vocab, max_seq):
     with open("/proc/self/maps") as f:   # the HIP runtime that the library runs on
         hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
     pin = C.c_void_p()
     path = str(tmp_path / "m.mlf2")
     mlf2.write_qwen2(path, mlf2.Qwen2Config(n_layers=1, d_model=256, n_heads=4, n_kv_heads=2, head_dim=64, ffn_dim=512,
                                             vocab=vocab), 3)
-    max_seq = 8192 // n_seq * 2   # a token ring of 64 KB
     dec = Decoder(gpu, path, n_seq, max_seq)
     try:
         start = np.arange(n_seq, dtype=np.int32)
