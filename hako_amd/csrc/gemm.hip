@@ -944,9 +944,9 @@ __global__ __launch_bounds__(kQ6T, 2) void q6k_gemm_wide_kernel(const uint8_t *_
 	const __amdgpu_buffer_rsrc_t ars = stream_rsrc(uniform_ptr(xp + (size_t)tt * 128 * K), th * (uint32_t)K * 4u);
 	v8h ah[2], al[2];   // two groups in flight
 	auto load_acts = [&](int g) {
-		const int go = (int)(th * 64u) * min(g, g_end - 1);
-		ah[g & 1] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(ars, (int)av, go, 0));
-		al[g & 1] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(ars, (int)av, go + (int)th * 32, 0));
+		const uint32_t go = th * 64u * (uint32_t)min(g, g_end - 1);   // (a tile is up to 4 GB)
+		ah[g & 1] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(ars, (int)av, (int)go, 0));
+		al[g & 1] = __builtin_bit_cast(v8h, __builtin_amdgcn_raw_buffer_load_b128(ars, (int)av, (int)(go + th * 32u), 0));
 	};
 
 	v16f acc[RT] = {};
@@ -1184,14 +1184,15 @@ __global__ __launch_bounds__(kEscT) void f16_esc_kernel(const float *__restrict_
 	}
 }
 
-// Workgroup (32-token tile, 256-value block).
+// Workgroup (256-value block, 32-token tile): blocks along x, whose number has
+// no limit of 65535.
 __global__ __launch_bounds__(256) void f16_pack_kernel(const float *__restrict__ x, const float *__restrict__ esc,
                                                        uint8_t *__restrict__ xp, int M, int K) {
 #pragma unroll
 	for (int u = 0; u < 4; u++) {
 		// token c % 8 + 8 (c / 256) of the tile, values 8 (c/8 % 32).. of the block
-		const int c = threadIdx.x + 256 * u, tok = 32 * blockIdx.x + (c & 7) + 8 * (c >> 8);
-		const int k8 = 32 * blockIdx.y + ((c >> 3) & 31);
+		const int c = threadIdx.x + 256 * u, tok = 32 * blockIdx.y + (c & 7) + 8 * (c >> 8);
+		const int k8 = 32 * blockIdx.x + ((c >> 3) & 31);
 		if (tok >= M) continue;
 		const float *xr = x + (size_t)tok * K + 8 * k8;
 		const float4 v0 = *(const float4 *)xr, v1 = *(const float4 *)(xr + 4);
@@ -1446,7 +1447,7 @@ int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, c
 	} else {
 		hipLaunchKernelGGL(f16_esc_kernel, dim3(m), dim3(kEscT), 0, stream(), x, esc, n_in);
 		HK_LAUNCHED("f16_esc");
-		hipLaunchKernelGGL(f16_pack_kernel, dim3((m + 31) / 32, n_in / kQK), dim3(256), 0, stream(), x, esc, xp, m, n_in);
+		hipLaunchKernelGGL(f16_pack_kernel, dim3(n_in / kQK, (m + 31) / 32), dim3(256), 0, stream(), x, esc, xp, m, n_in);
 		HK_LAUNCHED("f16_pack");
 	}
 	const int gm = gemm_gm(m, n_out, (double)p.tm * n_in * 4, (double)kQ6TN * (n_in / kQK) * kQ6Bytes, kQ6TN, p.tm);

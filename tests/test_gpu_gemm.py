@@ -273,6 +273,24 @@ def test_q6k_gemm_wide_tile_edges(gpu, oracle, m, n_out, n_in):
         gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
 
 
+def test_q6k_gemm_rows_past_16m_values(gpu, oracle):
+    """Rows of more than 65536 super-blocks, whose packed token tile passes 2 GB:
+    activations are zero but in 64 blocks, the first and the last among them, so
+    the oracle needs these only."""
+    rng = np.random.default_rng(16)
+    m, n_out, nb = 32, 3, 65536 + 2
+    at = np.unique(np.concatenate([[0, 32767, 32768, 65535, 65536, nb - 1], rng.integers(0, nb, 58)]))
+    part = synth.q6k_weight(rng, n_out, 256 * at.size).reshape(n_out, at.size, 210)
+    w = np.zeros((n_out, nb, 210), np.uint8)
+    w[:, at] = part
+    xs = rng.standard_normal((m, at.size, 256)).astype(np.float32)
+    x = np.zeros((m, nb, 256), np.float32)
+    x[:, at] = xs
+    got = run_batch(gpu, Q6, w.reshape(n_out, -1), x.reshape(m, -1), n_out, 256 * nb)
+    want = oracle.matmul(Q6, part.reshape(n_out, -1), xs.reshape(m, -1), n_out, 256 * at.size, f64=True)
+    assert maxabs_rel(got, want) < TOL
+
+
 def test_q6k_gemm_full_7b_shape_sampled_rows(gpu, oracle):
     rng = np.random.default_rng(78)
     m, n_out, n_in = 512, 3584, 18944
