@@ -1240,11 +1240,13 @@ int gemm_grid(int M, int N, int tn = kTN) {
 // Q4_K GEMM with K <= 3840: the resident-token-tile kernel (1) or the tiled
 // one (0); a launch-shape knob
 int g_q4_gemm_res = 1;
-// Q6_K GEMM in 256-row tiles of 64 or 128 tokens, or -1: by shape (a
-// launch-shape knob; the outputs of an unsplit K do not depend on it)
-int g_q6_gemm_tm = -1;
-// Split K in the Q6_K GEMM (0: one workgroup per tile)
-int g_q6_gemm_sk = 1;
+// Q6_K GEMM: 64- or 128-row tiles (tn), 256-row tiles of 64 or 128 tokens (tm), or
+// by shape (0). Launch-shape knobs: the outputs of an unsplit K are the same
+// bits in every form. tn goes before tm.
+int g_q6_gemm_tn = 0, g_q6_gemm_tm = 0;
+// Split K in 256-row tiles: in every entry point (2), in the decoder's prompt
+// pass only (1), never (0)
+int g_q6_gemm_sk = 2;
 
 int check_gemm(const char *what, int m, int n_out, int n_in, size_t row_bytes, const void *w) {
 	if (int rc = require_device()) return rc;
@@ -1260,8 +1262,10 @@ int check_gemm(const char *what, int m, int n_out, int n_in, size_t row_bytes, c
 }  // namespace
 
 void q4k_gemm_set_res(int v) { g_q4_gemm_res = v ? 1 : 0; }
-void q6k_gemm_set_tn(int v) { g_q6_gemm_tm = (v == 64 || v == 128) ? v : -1; }
-void q6k_gemm_set_sk(int v) { g_q6_gemm_sk = v > 0; }
+void q6k_gemm_set_tn(int v) { g_q6_gemm_tn = (v == 64 || v == 128) ? v : 0; }
+void q6k_gemm_set_tm(int v) { g_q6_gemm_tm = (v == 64 || v == 128) ? v : 0; }
+void q6k_gemm_set_sk(int v) { g_q6_gemm_sk = v < 0 ? 0 : (v > 2 ? 2 : v); }
+bool q6k_gemm_batch_splits() { return g_q6_gemm_sk == 2; }
 
 int q4k_gemm(float *y, const void *w, const int8_t *xq, const float *xs, const float *bias, int m, int n_out,
              int n_in) {
@@ -1366,7 +1370,7 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 		if (int rc = q6k_skinny(segs, kSkStore, xh, xl, esc, m, n_in, n_out, part, pf)) return rc;
 		return ok();
 	}
-	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, (float *)skp);
+	return q6k_gemm_x(y, w, x, ws, esc, bias, m, n_out, n_in, false, q6k_gemm_batch_splits() ? (float *)skp : nullptr);
 }
 
 namespace {
@@ -1390,9 +1394,10 @@ Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, bool room) {
 	Q6Plan best{};
 	const int small = ((m + kTM - 1) / kTM) * ((n_out + kTN - 1) / kTN);
 	double best_us = 8.5 + NB * (small <= cus ? 2.3 : 3.5 * ((small + 2 * cus - 1) / (2 * cus)));
-	if (g_q6_gemm_tm > 0) best_us = 1e30;
+	if (g_q6_gemm_tn) return best;
+	if (g_q6_gemm_tm) best_us = 1e30;
 	for (int tm = 128; tm >= 64; tm -= 64) {
-		if (g_q6_gemm_tm > 0 && tm != g_q6_gemm_tm) continue;
+		if (g_q6_gemm_tm && tm != g_q6_gemm_tm) continue;
 		Q6Plan p;
 		p.tm = tm;
 		p.tiles = ((m + tm - 1) / tm) * ((n_out + kQ6TN - 1) / kQ6TN);
@@ -1423,7 +1428,7 @@ int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, c
 		_Float16 *xh = (_Float16 *)act, *xl = xh + (size_t)m * n_in;
 		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 		// 128-row tiles when they still give about one workgroup per CU
-		const bool wide = 4 * (((m + kTM - 1) / kTM) * ((n_out + 127) / 128)) >= 3 * cu_count();
+		const bool wide = g_q6_gemm_tn ? g_q6_gemm_tn == 128 : 4 * (((m + kTM - 1) / kTM) * ((n_out + 127) / 128)) >= 3 * cu_count();
 		const int tn = wide ? 128 : kTN;
 		const int gm = gemm_gm(m, n_out, (double)kTM * n_in * 4, (double)tn * (n_in / kQK) * kQ6Bytes, tn);
 		if (wide)

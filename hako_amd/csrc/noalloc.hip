@@ -129,7 +129,8 @@ extern "C" int hako_gpu_matmul_batch_noalloc(float *y, const float *x, int type,
 	if (skinny) {
 		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
 		if (int rc = q6k_skinny(segs, kSkStore, xh, xl, esc, m, n_in, n_out, part, pf)) return rc;
-	} else if (int rc = q6k_gemm_x(y, w, x, base, esc, bias, m, n_out, n_in, false, (float *)(base + kScratchBytes))) {
+	} else if (int rc = q6k_gemm_x(y, w, x, base, esc, bias, m, n_out, n_in, false,
+	                               q6k_gemm_batch_splits() ? (float *)(base + kScratchBytes) : nullptr)) {
 		return rc;
 	}
 	return ok();

@@ -73,6 +73,7 @@ int q4k_gemm_segs(const SkSegs &segs, int epi, const int8_t *xq, const float *xs
 // (null: K stays whole).
 int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, const float *bias, int m, int n_out,
                int n_in, bool add, float *skp);
+bool q6k_gemm_batch_splits();   // whether the matmul entry points (not only the decoder) split K
 constexpr size_t kQ6SplitFloats = (size_t)256 * 128 * 256;   // of any launch: 256 workgroups of 128 x 256 sums
 
 }  // namespace hako

@@ -71,13 +71,14 @@ const char *hako_gpu_last_error(void);
 #define HAKO_TUNE_Q6K_FLAT_SEG  10   /* Q6_K flat grid, rows wider than 64 chunks: chunks per part, 64 or 32, or 0 = by shape (default) */
 #define HAKO_TUNE_Q6K_ROWS      11   /* Q6_K rows grid: 10 x waves + items in flight (44, 82, 84, 162), 0 = by shape (default), -1 = never */
 #define HAKO_TUNE_Q4K_GEMM_RES  12   /* Q4_K multi-token matmul with n_in <= 3840: 1 = resident token tile (default), 0 = 64 x 64 tiles */
-#define HAKO_TUNE_Q6K_GEMM_TN   13   /* Q6_K multi-token matmul: 256-row tiles of 64 or 128 tokens, or 0 = by shape, 64 x 64 tiles among them (default) */
+#define HAKO_TUNE_Q6K_GEMM_TN   13   /* Q6_K multi-token matmul: 64 x 64 or 64-token x 128-row tiles (64, 128), or 0 = by shape, 256-row tiles among them (default); the same bits where K is not split */
 #define HAKO_TUNE_Q6K_DIGITS    14   /* Q6_K persistent GEMV grid: 1 = integer activation columns (default), 0 = fp32 product per weight */
-#define HAKO_TUNE_Q6K_GEMM_SK   15   /* Q6_K multi-token matmul, 256-row tiles: K split over workgroups when the tiles leave CUs idle (1, 2; default 1), or never (0) */
+#define HAKO_TUNE_Q6K_GEMM_SK   15   /* Q6_K multi-token matmul in 256-row tiles, K split over workgroups when the tiles leave CUs idle: 2 = in every entry point (default), 1 = in the decoder's prompt pass only, 0 = never */
 #define HAKO_TUNE_DEC_GU_GRID   16   /* one-sequence decoder gate/up launch: 1 = flat grid, 2 = persistent grid (one workgroup per CU, the rmsnorm prologue once per workgroup), 0 = by shape (default: persistent); read when a step is enqueued or captured */
 #define HAKO_TUNE_DEC_MERGE_ROWS 17  /* one-sequence decoder merge+o launch: rows per workgroup, 64 or 128, or 0 = by shape (default: 128 past d_model 2048); the same bits either way; read when a step is enqueued or captured */
 #define HAKO_TUNE_DEC_QKV_ITEMS  18  /* one-sequence decoder q/k/v launch: row items per wave, 2, 4 or 8, or 0 = by shape (default: 8 past d_model 2048, else 2); the same bits either way; read when a step is enqueued or captured */
 #define HAKO_TUNE_DEC_ATTN_PARTS 19  /* one-sequence decoder attention: workgroups that share a query-head group, 1..8, or 0 = by shape (default: 2 with 7 heads per group, else up to 4); the same bits either way; read when a step is enqueued or captured */
+#define HAKO_TUNE_Q6K_GEMM_TM   20   /* Q6_K multi-token matmul: 256-row tiles of 64 or 128 tokens (HAKO_TUNE_Q6K_GEMM_TN goes before it), or 0 = by shape (default); the same bits where K is not split */
 int hako_gpu_tune(int knob, int value);
 
 typedef struct {

@@ -17,6 +17,7 @@ TOL = 1e-5
 Q4, Q6 = synth.TYPE_Q4_K, synth.TYPE_Q6_K
 HAKO_TUNE_Q6K_GEMM_TN = 13   # include/hako_gpu.h
 HAKO_TUNE_Q6K_GEMM_SK = 15
+HAKO_TUNE_Q6K_GEMM_TM = 20
 
 
 def run_batch(gpu, qtype, w, x, n_out, n_in, bias=None):
@@ -167,57 +168,64 @@ def test_q4k_gemm_full_7b_shape_sampled_rows(gpu, oracle):
         b.free()
 
 
-@pytest.mark.parametrize("m,n_out,n_in", [(64, 128, 256), (130, 200, 2048), (77, 3648, 1024), (512, 384, 4608)])
+@pytest.mark.parametrize("m,n_out,n_in", [(64, 128, 256), (130, 200, 2048), (77, 3648, 1024), (512, 384, 4608),
+                                         (17, 65, 768), (500, 3001, 512), (130, 9000, 768)])
 def test_q6k_gemm_tile_widths_agree_bit_exact(gpu, oracle, m, n_out, n_in):
-    """The 64-row and the 128-row (double-buffered) tiles do the same
-    arithmetic per output in the same order, so their outputs are
-    bit-identical, ragged token and row edges included; both within the bar
-    of the oracle. (Stream-K, which adds a tile's K pieces after the fact,
-    is off here and tested below.)"""
+    """The 64-row and the 128-row (double-buffered) tiles and the 256-row tiles
+    of 64 and 128 tokens do the same arithmetic per output in the same order
+    while K is not split, so their outputs are bit-identical, ragged token and
+    row edges included, and so is whichever of them the shape is given by
+    itself (64, 128 and 256 rows here); within the bar of the oracle."""
     rng = np.random.default_rng(m + n_out + n_in)
     w = synth.q6k_weight(rng, n_out, n_in)
     x = rng.standard_normal((m, n_in)).astype(np.float32)
     bias = 0.1 * rng.standard_normal(n_out).astype(np.float32)
     got = {}
-    gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 0)   # (the standalone call's default leaves it off too)
+    gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 0)
     try:
-        for tn in (64, 128):
+        for tn, tm in ((64, 0), (128, 0), (0, 64), (0, 128), (0, 0)):
             gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, tn)
-            got[tn] = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
+            gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, tm)
+            got[tn, tm] = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
     finally:
         gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0)
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
-    assert np.array_equal(got[64].view(np.uint32), got[128].view(np.uint32))
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2)
+    for form, y in got.items():
+        assert np.array_equal(y.view(np.uint32), got[64, 0].view(np.uint32)), form
     want = oracle.matmul(Q6, w, x, n_out, n_in, bias=bias, f64=True)
-    assert maxabs_rel(got[128], want) < TOL
+    assert maxabs_rel(got[128, 0], want) < TOL
 
 
+@pytest.mark.parametrize("tm", [64, 128])
 @pytest.mark.parametrize("m,n_out,n_in", [(130, 200, 2048), (77, 3648, 1024), (512, 384, 4608), (64, 128, 512),
                                          (512, 3584, 4608)])
-def test_q6k_gemm_stream_k(gpu, oracle, m, n_out, n_in):
-    """128-row tiles in stream-K form (every CU takes an equal share of the
-    tiles' super-blocks; a tile's pieces meet in a second launch, in order of
-    K) against the same tiles whole: within 1e-6, and the GEMM bar of the
-    oracle. The shapes give tiles held by one to several workgroups, pieces
-    of one super-block, ragged token and row edges; twice in a row, the
-    second call on other inputs, so no stale slot passes."""
+def test_q6k_gemm_split_k(gpu, oracle, m, n_out, n_in, tm):
+    """256-row tiles whose K is split over workgroups (a tile's ranges of its
+    super-blocks meet in a second launch, in order of K) against the same
+    tiles whole: within 1e-6, and the GEMM bar of the oracle. The shapes give
+    tiles of one to many workgroups, ranges of one super-block and of unequal
+    length, ragged token and row edges; twice in a row, the second call on
+    other inputs, so no stale sum passes. With the knob at 1 only the decoder
+    splits."""
     rng = np.random.default_rng(3 * m + n_out + n_in)
     w = synth.q6k_weight(rng, n_out, n_in)
     bias = 0.1 * rng.standard_normal(n_out).astype(np.float32)
-    gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 128)
+    gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, tm)
     try:
         for call in range(2):
             x = rng.standard_normal((m, n_in)).astype(np.float32) * (1.0 + 9.0 * call)
-            gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 0)
-            whole = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
-            gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2)
-            got = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
-            assert maxabs_rel(got, whole) < 1e-6
+            got = {}
+            for sk in (0, 1, 2):
+                gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, sk)
+                got[sk] = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
+            assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+            assert maxabs_rel(got[2], got[0]) < 1e-6
             want = oracle.matmul(Q6, w, x, n_out, n_in, bias=bias, f64=True)
-            assert maxabs_rel(got, want) < TOL
+            assert maxabs_rel(got[2], want) < TOL
     finally:
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0)
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2)
 
 
 @pytest.mark.parametrize("m,n_out,n_in", [(17, 1, 512), (32, 33, 768), (33, 65, 2048), (77, 2048, 2048),
@@ -263,14 +271,14 @@ def test_q6k_gemm_wide_tile_edges(gpu, oracle, m, n_out, n_in):
     scale = np.max(np.abs(want), axis=1, keepdims=True)
     try:
         for tm in (64, 128):
-            gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, tm)
-            for sk in (0, 1):
+            gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, tm)
+            for sk in (0, 2):
                 gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, sk)
                 got = run_batch(gpu, Q6, w, x, n_out, n_in, bias)
                 assert np.max(np.abs(got - want) / scale) < TOL
     finally:
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0)
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2)
 
 
 def test_q6k_gemm_rows_past_16m_values(gpu, oracle):

@@ -187,14 +187,14 @@ def test_prefill_matches_reference_feed(gpu, ref, tmp_path, cfg, seed, n_prompt,
         assert max(err_k, err_v) <= 2 * err_nf
 
 
-HAKO_TUNE_Q6K_GEMM_TN, HAKO_TUNE_Q6K_GEMM_SK = 13, 15
+HAKO_TUNE_Q6K_GEMM_TM, HAKO_TUNE_Q6K_GEMM_SK = 20, 15
 
 
-def test_prefill_stream_k_down_matches_reference_feed(gpu, ref, tmp_path):
-    """The down projection's Q6_K GEMM in its stream-K form inside the prompt
-    pass (128-row tiles forced: 3 x 8 tiles of 11 super-blocks over the
-    grid, so every tile's K is split over many workgroups and the fixup adds
-    the pieces into the residual) against whole tiles and the reference's
+def test_prefill_split_k_down_matches_reference_feed(gpu, ref, tmp_path):
+    """The down projection's Q6_K GEMM with K split over workgroups inside the
+    prompt pass (tiles of 128 tokens x 256 rows forced: 2 x 4 tiles of 11
+    super-blocks, so that a tile's K is shared by up to 11 workgroups and a
+    second launch adds the pieces into the residual) against whole tiles and the reference's
     feed: the same greedy tokens, K/V rows and logits within the bars of the
     SMALL_128 case above."""
     cfg, seed, n_prompt, max_seq = SMALL_128, 21, 140, 384
@@ -210,7 +210,7 @@ def test_prefill_stream_k_down_matches_reference_feed(gpu, ref, tmp_path):
     finally:
         r.close()
     got = {}
-    gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 128)
+    gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 128)
     try:
         for sk in (0, 1):
             gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, sk)
@@ -224,12 +224,12 @@ def test_prefill_stream_k_down_matches_reference_feed(gpu, ref, tmp_path):
                 dec.close()
             got[sk] = (lg, k, v, toks)
     finally:
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0)
-        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 1)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2)
     for sk, (lg, k, v, toks) in got.items():
-        within(f"stream-K {sk} K", k, want_k, 3.8e-4)
-        within(f"stream-K {sk} V", v, want_v, 3.8e-4)
-        within(f"stream-K {sk} logits", lg, want_lg, 3e-6)
+        within(f"split K {sk} K", k, want_k, 3.8e-4)
+        within(f"split K {sk} V", v, want_v, 3.8e-4)
+        within(f"split K {sk} logits", lg, want_lg, 3e-6)
         assert toks == want, sk
 
 
