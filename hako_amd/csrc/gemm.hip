@@ -1376,29 +1376,36 @@ int q6k_gemm(float *y, const void *w, const float *x, const float *bias, int m, 
 namespace {
 
 // The launch of m x n_out x n_in, with room for the sums of a split K or
-// without: the 64- or 128-row tiles (tm = 0), or tm tokens x 256 rows and the
-// workgroups that share a tile's K (no more than the CUs take at once, one
-// workgroup per CU: registers and 80 KB of LDS; and no more sums than
+// without: tiles of 64 tokens x tn (64, 128) rows, or (tn = 0) of tm tokens x 256
+// rows and the workgroups that share a tile's K (no more than the CUs take at
+// once, one workgroup per CU: registers and 80 KB of LDS; and no more sums than
 // kQ6SplitFloats, which every caller's room holds, so that all of them split
-// alike and give the same bits). Chosen by what each would take: per super-block 2.3 us (one tile per
-// CU) or 3.5 us per round of two for the 64-row tiles, 8.7 and 6.0 us for 128
-// and 64 tokens, the sums of a split K written and read at 4 TB/s, and a start
-// of 8.5 and 9 us. Within 25% of what 64 shapes measured (17 .. 512 tokens, 64
-// .. 18944 rows, 256 .. 2048 values: q6_k 4096 x 512 at 200 tokens 12.4 us in
-// small tiles and 19.2 in wide ones, 18944 x 512 at 200 tokens 32.4 and 27.0).
+// alike and give the same bits). Chosen by what each would take: a start of 8.5
+// us, and per super-block 2.15 us (one tile per CU) or 3.4 us per round of two
+// for the 64-row tiles, 3.25 us per round of one for the 128-row ones, 8.7 and
+// 6.0 us for 128 and 64 tokens x 256 rows, and the sums of a split K written and
+// read at 4 TB/s. Measured in every form at 1170 shapes (17 .. 512 tokens, 64 ..
+// 18944 rows, 256 .. 18944 values): the chosen one is on average 0.6% from the
+// fastest and nowhere slower than the better of 64- and 128-row tiles by their
+// old rule (128 rows for three quarters of the CUs or more). 4608 x 512 at 200
+// tokens 13.9 us in 128-row tiles, 15.3 in 64-row, 19.4 in 256-row ones, 18944 x
+// 512 at 200 tokens 31.2, 29.0 and 27.3, 3584 x 2048 at 77 tokens 33.1, 26.4 and
+// 27.6.
 struct Q6Plan {
-	int tm, tiles, ks;
+	int tn, tm, tiles, ks;
 };
 Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, bool room) {
 	const int NB = n_in / kQK, cus = cu_count();
+	const int mt = (m + kTM - 1) / kTM, t64 = mt * ((n_out + 63) / 64), t128 = mt * ((n_out + 127) / 128);
+	const double us64 = 8.5 + NB * (t64 <= cus ? 2.15 : 3.4 * ((t64 + 2 * cus - 1) / (2 * cus)));
+	const double us128 = 8.5 + NB * 3.25 * ((t128 + cus - 1) / cus);
 	Q6Plan best{};
-	const int small = ((m + kTM - 1) / kTM) * ((n_out + kTN - 1) / kTN);
-	double best_us = 8.5 + NB * (small <= cus ? 2.3 : 3.5 * ((small + 2 * cus - 1) / (2 * cus)));
+	best.tn = g_q6_gemm_tn ? g_q6_gemm_tn : us128 < us64 ? 128 : 64;
 	if (g_q6_gemm_tn) return best;
-	if (g_q6_gemm_tm) best_us = 1e30;
+	double best_us = g_q6_gemm_tm ? 1e30 : best.tn == 128 ? us128 : us64;
 	for (int tm = 128; tm >= 64; tm -= 64) {
 		if (g_q6_gemm_tm && tm != g_q6_gemm_tm) continue;
-		Q6Plan p;
+		Q6Plan p{};
 		p.tm = tm;
 		p.tiles = ((m + tm - 1) / tm) * ((n_out + kQ6TN - 1) / kQ6TN);
 		const int most = !room || !g_q6_gemm_sk || cus < 2 * p.tiles ? 1 : cus / p.tiles < NB ? cus / p.tiles : NB;
@@ -1406,7 +1413,7 @@ Q6Plan q6k_gemm_plan(int m, int n_out, int n_in, bool room) {
 			const size_t slots = (size_t)p.tiles * p.ks * q6w_slot(tm);
 			if (p.ks > 1 && slots > kQ6SplitFloats) break;
 			const int rounds = p.ks > 1 ? 1 : (p.tiles + cus - 1) / cus;
-			const double us = 9.0 + rounds * ((NB + p.ks - 1) / p.ks) * (tm == 128 ? 8.7 : 6.0) +
+			const double us = 8.5 + rounds * ((NB + p.ks - 1) / p.ks) * (tm == 128 ? 8.7 : 6.0) +
 			                  (p.ks > 1 ? 4.0 + (double)slots * 8 / 4e6 : 0.0);
 			if (us < best_us) {
 				best = p;
@@ -1424,14 +1431,11 @@ int q6k_gemm_x(float *y, const void *w, const float *x, void *act, float *esc, c
 	if (int rc = check_gemm("Q6_K GEMM", m, n_out, n_in, (size_t)n_in / kQK * kQ6Bytes, w)) return rc;
 	if (m <= kSkMaxTokens) return set_error(HAKO_GPU_EINVAL, "Q6_K GEMM tiles need m > %d", kSkMaxTokens);
 	const Q6Plan p = q6k_gemm_plan(m, n_out, n_in, skp != nullptr);
-	if (!p.tm) {
+	if (p.tn) {
 		_Float16 *xh = (_Float16 *)act, *xl = xh + (size_t)m * n_in;
 		if (int rc = f16_split(x, xh, xl, esc, m, n_in)) return rc;
-		// 128-row tiles when they still give about one workgroup per CU
-		const bool wide = g_q6_gemm_tn ? g_q6_gemm_tn == 128 : 4 * (((m + kTM - 1) / kTM) * ((n_out + 127) / 128)) >= 3 * cu_count();
-		const int tn = wide ? 128 : kTN;
-		const int gm = gemm_gm(m, n_out, (double)kTM * n_in * 4, (double)tn * (n_in / kQK) * kQ6Bytes, tn);
-		if (wide)
+		const int gm = gemm_gm(m, n_out, (double)kTM * n_in * 4, (double)p.tn * (n_in / kQK) * kQ6Bytes, p.tn);
+		if (p.tn == 128)
 			hipLaunchKernelGGL((q6k_gemm_kernel<128, true>), dim3(gemm_grid(m, n_out, 128)), dim3(4 * 128),
 			                   2 * q6g_buf_bytes(128), stream(), (const uint8_t *)w, xh, xl, esc, bias, y, m, n_out, n_in,
 			                   add ? 1 : 0, gm);

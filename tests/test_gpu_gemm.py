@@ -175,7 +175,7 @@ def test_q6k_gemm_tile_widths_agree_bit_exact(gpu, oracle, m, n_out, n_in):
     of 64 and 128 tokens do the same arithmetic per output in the same order
     while K is not split, so their outputs are bit-identical, ragged token and
     row edges included, and so is whichever of them the shape is given by
-    itself (64, 128 and 256 rows here); within the bar of the oracle."""
+    itself (64 and 128 rows here); within the bar of the oracle."""
     rng = np.random.default_rng(m + n_out + n_in)
     w = synth.q6k_weight(rng, n_out, n_in)
     x = rng.standard_normal((m, n_in)).astype(np.float32)
