@@ -296,10 +296,13 @@ __global__ __launch_bounds__(kGT, 3) void q4k_gemm_kernel(const SkSegs segs, con
 // With few units per workgroup (a short prompt, a small matrix) most waves
 // would have none, and the others a serial chain over the whole K: KW lets kw
 // waves share a unit, a range of K each, their sums meeting in LDS in order of
-// K. 2048 x 2048 at 77 tokens (one unit per workgroup, 8 waves each) 17.2 ->
-// 12.5 us, 2048 x 3584 at 200 tokens (three) 26.0 -> 19.2; from four units on
-// only where K is long (2048 x 1024 at 512 tokens 15.5 -> 16.3, x 3584 30.6 ->
-// 28.5). One wave per unit is its own instance: the two in one spill registers.
+// K. With its q8 launch, 2048 x 2048 at 77 tokens (one unit per workgroup, 8
+// waves each) 17.1 -> 11.3 us, 2048 x 3584 at 200 tokens (two, 6 waves) 25.7 ->
+// 18.0; three and four units only where K is longer than 2 super-blocks per unit
+// (four: 2048 x 3584 at 512 tokens 30.0 -> 26.9, x 1024 15.5 -> 16.3 when
+// tried), five and more never. The sums' order, and so a token's last bits,
+// then depends on how many tokens the call has. One wave per unit is its own
+// instance: the two in one spill registers.
 // Grid: token tiles x R row ranges, in XCD-contiguous order with the token
 // tiles minor: the workgroups of one XCD share a row range, whose weights
 // then come from that XCD's L2 after the first read.
@@ -1021,7 +1024,6 @@ __global__ __launch_bounds__(kQ6T, 2) void q6k_gemm_wide_kernel(const uint8_t *_
 	load_acts(16 * ka + 1);
 	// Stage st is in buffer st % 2, stored before the barrier that ends
 	// stage st - 1, after the barrier that ended the buffer's last reader.
-	// #pragma unroll
 	for (int i = 0; i < 8; i++) conv_wts(b0, 0, i);
 	conv_scales(b0, 0, 0);
 	__syncthreads();

@@ -201,7 +201,9 @@ int hako_gpu_q6k_gemm(float *y, const void *w, const float *x, const float *bias
 /* matmul over m activation rows for any supported type: Q4_K quantizes the
  * rows with the q8_32 scheme (library workspace) then runs the Q4_K GEMM;
  * Q6_K runs the Q6_K GEMM; F32/F16 run one GEMV per row; m == 1 is
- * hako_gpu_matmul. */
+ * hako_gpu_matmul. A call repeats itself bit for bit. Between calls of
+ * different m, a token's outputs may differ in their last bits: the tiles, and
+ * with them the order in which its fp32 sums are added, follow the shape. */
 int hako_gpu_matmul_batch(float *y, const float *x, int type, const void *w,
                           const float *bias, int m, int n_out, int n_in);
 

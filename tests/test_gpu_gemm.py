@@ -229,11 +229,12 @@ def test_q6k_gemm_split_k(gpu, oracle, m, n_out, n_in, tm):
 
 
 @pytest.mark.parametrize("m,n_out,n_in", [(17, 1, 512), (32, 33, 768), (33, 65, 2048), (77, 2048, 2048),
-                                         (77, 4608, 1280), (200, 3000, 3584), (512, 2048, 3840), (512, 2048, 2048)])
+                                         (77, 4608, 1280), (200, 3000, 3584), (512, 2048, 3840), (512, 2048, 2048),
+                                         (64, 512, 3584), (200, 2048, 3584)])
 def test_q4k_gemm_shared_units(gpu, oracle, m, n_out, n_in):
-    """Few 32-row units per workgroup, so that several waves share one (from
-    two waves of one super-block each to twelve, and fewer super-blocks than
-    waves); the last shape is the first past the rule. Integer inputs with one
+    """Few 32-row units per workgroup, so that several waves share one: 2, 3, 8,
+    8, 5, 4, 3, 1 (the first shape past the rule), 12 and 6 of them, some with
+    fewer super-blocks than waves. Integer inputs with one
     (s, m) = (1, 0) per block and unit scales: every output is exact in
     fp32 whatever the order of the sums."""
     rng = np.random.default_rng(m + n_out + n_in)
