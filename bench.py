@@ -573,6 +573,10 @@ def main():
         sys.exit(2)
 
     from hako_amd.gpu import Gpu
+    from oracle.hako_oracle import REF_LIB
+    if not args.no_cpu and not os.path.exists(REF_LIB):
+        log("no CPU baselines: the reference library is not built (its sources are absent)")
+        args.no_cpu = True
     g = Gpu(0)
     info = g.info()
     log(f"device {info.name.decode()} CUs={info.compute_units} HBM={info.hbm_bytes / 2**30:.0f} GiB")
