@@ -22,6 +22,15 @@ def oracle():
 
 
 @pytest.fixture(scope="session")
+def compiled_reference():
+    """Skips where the reference's sources, and so the libraries that oracle/ref.mk builds from them, are absent."""
+    from oracle.hako_oracle import REF_LIB, REF_MODEL_LIB, REF_NOFAST_LIB
+    for lib in (REF_LIB, REF_MODEL_LIB, REF_NOFAST_LIB):
+        if not os.path.exists(lib):
+            pytest.skip(f"reference library not built: {os.path.basename(lib)}")
+
+
+@pytest.fixture(scope="session")
 def golden():
     cache = {}
 

@@ -70,7 +70,7 @@ def test_mlf2_writer_layout(tmp_path):
     assert emb.size == 512 * 210
 
 
-def test_reference_loads_and_runs_written_model(tmp_path):
+def test_reference_loads_and_runs_written_model(tmp_path, compiled_reference):
     """The reference's own mlf2_open / hakm_ctx_new / hakm_forward (CPU)
     accept the synthetic file and produce finite logits."""
     from oracle.hako_oracle import REF_LIB
@@ -85,7 +85,7 @@ def test_reference_loads_and_runs_written_model(tmp_path):
     assert len(toks) == 3 and np.all(np.isfinite(logits))
 
 
-def test_host_elementwise_helpers_match_reference():
+def test_host_elementwise_helpers_match_reference(compiled_reference):
     """rmsnorm / softmax / silu_f / rope_neox of libhako.so (host code) against
     the reference's compiled nn.c."""
     from oracle.hako_oracle import REF_LIB

@@ -39,7 +39,7 @@ GQA2 = mlf2.Qwen2Config(n_layers=2, d_model=512, n_heads=8, n_kv_heads=4, head_d
 
 
 @pytest.fixture(scope="module")
-def ref():
+def ref(compiled_reference):
     from dropin import bind_ctx
     from oracle.hako_oracle import REF_LIB
     return bind_ctx(C.CDLL(REF_LIB))
@@ -481,7 +481,7 @@ def test_non_finite_values_follow_reference(gpu, ref, tmp_path, name, where, val
 
 
 @pytest.fixture(scope="module")
-def ref_nofast():
+def ref_nofast(compiled_reference):
     """The reference's sources built without -ffast-math (oracle/ref.mk): a
     second correct build, whose drift from the first measures how much a
     model amplifies differences in rounding order."""

@@ -89,7 +89,7 @@ TINY_UNTIED = mlf2.Qwen2Config(n_layers=2, d_model=512, n_heads=8, n_kv_heads=2,
 
 
 @pytest.mark.parametrize("cfg,seed", [(TINY, 1), (TINY_UNTIED, 2)])
-def test_reference_model_c_on_dropin(host, tmp_path, cfg, seed):
+def test_reference_model_c_on_dropin(host, compiled_reference, tmp_path, cfg, seed):
     """The reference's hakm_forward, unchanged, calling this library's matmul."""
     from dropin import bind_ctx, greedy
     from oracle.hako_oracle import REF_LIB, REF_MODEL_LIB
@@ -106,7 +106,7 @@ def test_reference_model_c_on_dropin(host, tmp_path, cfg, seed):
 
 
 @pytest.mark.timeout(600)
-def test_reference_model_c_on_dropin_qwen2_3b(host, tmp_path):
+def test_reference_model_c_on_dropin_qwen2_3b(host, compiled_reference, tmp_path):
     """The reference's hakm_forward, unchanged (src/model.c:93-165), on the
     full Qwen2.5-3B shape from a cache prefilled to 1024 positions, its 253
     matmuls per token through this library: two greedy steps give the

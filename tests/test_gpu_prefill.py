@@ -33,7 +33,7 @@ DENSE = mlf2.Qwen2Config(n_layers=1, d_model=256, n_heads=2, n_kv_heads=1, head_
 
 
 @pytest.fixture(scope="module")
-def ref():
+def ref(compiled_reference):
     from dropin import bind_ctx
     from oracle.hako_oracle import REF_LIB
     return bind_ctx(C.CDLL(REF_LIB))

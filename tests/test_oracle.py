@@ -169,7 +169,7 @@ def q8_non_finite_rows() -> np.ndarray:
     return rows
 
 
-def test_q8_non_finite_matches_compiled_reference(oracle):
+def test_q8_non_finite_matches_compiled_reference(oracle, compiled_reference):
     """NaN and infinite inputs: the oracle's codes and scales against the
     reference's compiled quantize_row_q8_32 (a NaN never enters the block
     maximum; a non-finite product converts to code 0; an infinite maximum
@@ -268,7 +268,7 @@ def test_argmax_lowest_index_wins(oracle):
     assert oracle.argmax(v) == 1
 
 
-def test_greedy_pick_non_finite_rules(oracle):
+def test_greedy_pick_non_finite_rules(oracle, compiled_reference):
     """The reference's compiled greedy pick (src/sample.c:28-31) and the
     oracle's agree on the non-finite rules the device argmax follows: a NaN
     at index 0 is kept, a NaN elsewhere never wins, ties go to the lowest
