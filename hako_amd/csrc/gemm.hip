@@ -626,10 +626,10 @@ constexpr int kHPad = kQ6Stage + 8;  // fp16 per staged row (272 B: conflict-fre
 
 // ── Q6_K x fp32, 64- and 128-row tiles ──
 //
-// For short K (q6k_gemm_plan): their start-up is the shortest (10 against 14
-// us at 512 x 64 x 256 with the split of the activations, 25 against 34 at
-// 512 x 4096 x 1024), their cost per super-block the highest (273 against 192 us
-// at 512 x 3584 x 18944).
+// For short K (q6k_gemm_plan): their start-up is the shortest (10 against 12
+// us at 512 x 64 x 256 with the split of the activations, 14 against 19 at 200
+// x 4608 x 512), their cost per super-block the highest (266 against 192 us at
+// 512 x 3584 x 18944).
 //
 // LDS of one stage buffer of a TN-row tile: activation hi and lo
 // [64][kHPad], q - 32 [TN][kHPad] (fp16), d*sc [8 groups][TN] (fp32).
