@@ -187,7 +187,7 @@ def test_prefill_matches_reference_feed(gpu, ref, tmp_path, cfg, seed, n_prompt,
         assert max(err_k, err_v) <= 2 * err_nf
 
 
-HAKO_TUNE_Q6K_GEMM_TM, HAKO_TUNE_Q6K_GEMM_SK = 20, 15
+HAKO_TUNE_Q4K_GEMM_RES, HAKO_TUNE_Q6K_GEMM_TN, HAKO_TUNE_Q6K_GEMM_SK, HAKO_TUNE_Q6K_GEMM_TM = 12, 13, 15, 20
 
 
 def test_prefill_split_k_down_matches_reference_feed(gpu, ref, tmp_path):
@@ -231,6 +231,52 @@ def test_prefill_split_k_down_matches_reference_feed(gpu, ref, tmp_path):
         within(f"split K {sk} V", v, want_v, 3.8e-4)
         within(f"split K {sk} logits", lg, want_lg, 3e-6)
         assert toks == want, sk
+
+
+SHARED = mlf2.Qwen2Config(n_layers=2, d_model=1536, n_heads=12, n_kv_heads=2, head_dim=128, ffn_dim=2304,
+                          vocab=512, ctx=256)
+
+
+@pytest.mark.parametrize("n_prompt", [40, 77, 150])
+def test_prefill_shared_units_and_split_k_match_whole_k(gpu, tmp_path, n_prompt):
+    """Every Q4_K product of a block with its units shared by waves (three
+    segments of q/k/v, the residual added after o, SwiGLU rows: 6 waves per
+    unit, for 150 tokens one in gate/up) and the down projection's K split
+    over workgroups, against the 64 x 64 tiles with whole K. The first block's
+    keys and values have the same 8-bit inputs, so they differ by the order of
+    fp32 sums only. What comes after may differ where a value lies next to
+    an edge of the 8-bit rounding: one code that flips moves a row by about
+    amax / 127 of one of 1536 inputs, 0.02 / sqrt(1536) = 5e-4 of its rms and
+    less of its largest value, and a row has 0.03 of them on average (inputs
+    apart by 2e-7 of their rms). A unit or a range of K missed or taken twice
+    moves it by 0.1 and more."""
+    path = str(tmp_path / "m.mlf2")
+    mlf2.write_qwen2(path, SHARED, 23)
+    prompt = np.random.default_rng(n_prompt).integers(0, SHARED.vocab, n_prompt).astype(np.int32)
+    got = {}
+    try:
+        for shared in (0, 1):
+            gpu.tune(HAKO_TUNE_Q4K_GEMM_RES, shared)
+            gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0 if shared else 64)
+            gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 64 if shared else 0)
+            gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2 * shared)
+            dec = make(gpu, path, 1, 256)
+            try:
+                dec.set_pos(0)
+                _, lg = dec.prefill(prompt, logits=True)
+                got[shared] = lg, *device_kv(gpu, dec, 0, n_prompt)
+            finally:
+                dec.close()
+    finally:
+        gpu.tune(HAKO_TUNE_Q4K_GEMM_RES, 1)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TN, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_TM, 0)
+        gpu.tune(HAKO_TUNE_Q6K_GEMM_SK, 2)
+    (lg0, k0, v0), (lg1, k1, v1) = got[0], got[1]
+    for name, a, b in (("K", k1, k0), ("V", v1, v0)):
+        within(f"first block {name}", a[0], b[0], 1e-6)
+        within(f"second block {name}", a[1], b[1], 2e-3)
+    within("logits", lg1, lg0, 2e-3)
 
 
 # head_dim 64 takes the chunk-record attention, head_dim 128 (SMALL_128) the
